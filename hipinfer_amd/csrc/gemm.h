@@ -14,8 +14,13 @@
 //    while the MFMAs consume the current one;
 //  * within a tile the fragments of step s+1 are read from LDS while the MFMAs of step s run (the
 //    order is pinned with scheduling-group barriers: MFMA, LDS read, MFMA, ...); the one barrier
-//    per tile sits in the last step, after its fragments are in registers, and is followed at once
-//    by the DMA that refills the stage just freed and by the first fragment reads of the next tile.
+//    per tile sits before the last step, after its fragments are in registers, and frees the tile's
+//    stage. The DMA that refills it goes out in parts behind the MFMAs of the following steps: issued
+//    in one burst after the barrier, a wave's 8-16 DMA instructions held up its own MFMAs while the
+//    CU's L1 path (64 B per clock) worked through 64 KB. Measured on one card each, cold weights,
+//    burst -> parts: M = 2048, N = 28672, K = 4096 (256 x 256) 440 -> 416 us; M = 2048, N = 4096,
+//    K = 14336 (256 x 128) 236 -> 217; M = 1000, N = 5120, K = 3072 (128 x 160) 41.4 -> 39.0; int8
+//    M = 333, N = 17920, K = 1536 32.4 -> 30.8; M = 512, N = 11264, K = 2048 34.3 -> 31.4.
 //    The refill is unconditional (past the split's last tile it re-reads the first), so the loop
 //    body has no branch and its DMA waits are compile-time counts;
 //  * LDS rows hold 16-byte chunks at positions XOR-swizzled by the row (c ^ ((r >> 1) & 7) for
@@ -43,6 +48,8 @@
 //    partials visible across XCDs; an in-kernel "last block reduces" handoff would need an
 //    agent-scope fence, which writes back and invalidates the XCD's L2 on this part.
 #pragma once
+#include <type_traits>
+
 #include "hi_common.h"
 
 struct GemmArgs {
@@ -121,22 +128,32 @@ __device__ __forceinline__ int lds_off8(int r, int c) {
   else return r * 32 + ((c ^ ((r >> 3) & 1)) << 4);
 }
 
-// Scheduling pattern of one step: the step's NM MFMAs alternate with the ND LDS reads of the next
-// step's fragments (then whichever is left over), so the reads are issued early and their latency
-// hides under the matrix work instead of being sunk next to their first use.
-template <int NM, int ND>
+// Scheduling pattern of one step: behind each of the step's NM MFMAs one of the ND LDS reads of the
+// next step's fragments, then the NV DMA instructions of the refill under way, spread over the MFMAs
+// left (then whichever is left over). The reads are issued early and their latency hides under the
+// matrix work instead of being sunk next to their first use, and no DMA instruction queues up
+// behind another one in front of the MFMAs.
+template <int NM, int ND, int NV = 0>
 __device__ __forceinline__ void sched_step() {
-  constexpr int P = ND < NM ? ND : NM;
+  constexpr int P = ND < NM ? ND : NM, R = NM - P;  // MFMAs before and after the last read
 #pragma unroll
   for (int i = 0; i < P; i++) {
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
   }
-  if constexpr (NM > P) __builtin_amdgcn_sched_group_barrier(0x008, NM - P, 0);
   if constexpr (ND > P) __builtin_amdgcn_sched_group_barrier(0x100, ND - P, 0);
+  int v = 0;
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#pragma unroll
+    for (; v * R < (i + 1) * NV; v++) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // DMA
+  }
+#pragma unroll
+  for (; v < NV; v++) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
 }
 
-template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, bool GRP = false, int BK = 64, int KG = 1>
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, bool GRP = false, int BK = 64, int KG = 1, int SB = S>
 __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
   constexpr int TM = BM / WM, TN = BN / WN;          // wave tile
   constexpr int FM = TM / 32, FN = TN / 32;          // MFMA tiles per wave
@@ -149,9 +166,27 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
   constexpr int A_LD = BM * 2 * BK / 1024 / NW;      // 1 KB DMA instructions per wave per K tile (A)
   constexpr int B_LD = BN * B_ROWB / 1024 / NW;      // ... (W)
   constexpr int L = A_LD + B_LD;                     // vector-memory ops per lane per K tile
+  // A refill (one K tile of A and of W into the stages just freed) is issued in NP parts, one per
+  // step of MFMAs after the barrier that freed them, so that no wave's DMA instructions queue up
+  // behind one another in front of its MFMAs. A two-stage ring has no tile of slack and issues it in
+  // the first step; one with a third W stage takes A first, in two steps, W then has a tile more to
+  // land. Other rings take W first (cold weights come from HBM, the activations mostly from L2).
+  constexpr int NP = SB == 2 ? 1 : BK == 32 || S == 2 || GRP ? 2 : 4;
+  constexpr auto part_n = [](int p) constexpr {
+    int n = 0;
+    for (int i = 0; i < L; i++) n += i * NP / L == p;
+    return n;
+  };
+  // the v-th instruction of part p, as an index for issue_one (A first)
+  constexpr auto part_at = [](int p, int v) constexpr {
+    int i = 0;
+    while (i * NP / L != p) i++;
+    i += v;
+    return SB == S ? (i + A_LD) % L : i;
+  };
   static_assert((NW == 4 || NW == 8) && FM >= 1 && FN >= 1 && TM % 32 == 0 && TN % 32 == 0, "wave tiling");
   static_assert(A_LD >= 1 && B_LD >= 1 && A_LD * 1024 * NW == BM * 2 * BK && B_LD * 1024 * NW == BN * B_ROWB &&
-                    S >= 2 && S <= 8 && (S - 1) * L < 64 && 3 * L < 64,
+                    S >= 2 && S <= 8 && (SB == S || SB == S + 1) && (S - 1) * L + B_LD < 64 && 3 * L < 64,
                 "pipeline shape: every wave issues the same whole number of 1 KB DMA instructions");
   static_assert(!(GRP && Q8), "grouped (expert) GEMMs take fp16 weights");
   static_assert(BK == 128 || BK == 64 || BK == 32, "K tile depth");
@@ -164,10 +199,10 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
   // each with its own S-stage ring; group 0 adds the other groups' sums at the end
   const int tid = threadIdx.x, lane = tid & 63;
   const int kg = KG > 1 ? (tid >> 6) / NW : 0;  // this wave's K group
-  const int wave = (tid >> 6) - kg * NW;        // its index within the group
-  f16* smem = reinterpret_cast<f16*>(smem_raw) + kg * S * (A_ST + B_ST);
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) - kg * NW);  // its index within the group
+  f16* smem = reinterpret_cast<f16*>(smem_raw) + kg * (S * A_ST + SB * B_ST);
   f16* As = smem;               // [S][BM][64]
-  f16* Bs = smem + S * A_ST;    // [S][BN][64] fp16, or [S][BN][64 bytes] int8
+  f16* Bs = smem + S * A_ST;    // [SB][BN][64] fp16, or [SB][BN][64 bytes] int8
 
   const int wm = wave / WN, wn = wave % WN;
   const int N = g.N, K = g.K;
@@ -278,30 +313,29 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
         a_go[i] = a_lo[(ri / RPI) % (BK == 128 ? 4 : 2)] + (int)((int64_t)ri * g.lda * 2);
     }
   }
-  auto issue = [&](int kt, int st) {
-    const int k0 = kt * BK;
-    f16* as = As + st * A_ST;
-#pragma unroll
-    for (int i = 0; i < A_LD; i++) {
+  // one DMA instruction of K tile kt_a / kt_b: A instruction i < A_LD into A stage sa, W
+  // instruction i - A_LD into W stage sb
+  auto issue_one = [&](int i, int kt_a, int sa, int kt_b, int sb) {
+    if (i < A_LD) {
+      const int k0 = kt_a * BK;
+      f16* as = As + sa * A_ST;
       const int ri = (wave * A_LD + i) * RPI;
       // (a plain conditional: an `if constexpr` here kept clang from emitting the grouped kernels)
-      const int off = GRP ? a_go[i] : a_lo[(ri / RPI) % (BK == 128 ? 4 : 2)] + (int)((int64_t)ri * g.lda * 2);
+      const int off = GRP ? a_go[i < A_LD ? i : 0] : a_lo[(ri / RPI) % (BK == 128 ? 4 : 2)] + (int)((int64_t)ri * g.lda * 2);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rs, (lds_void_t*)(as + ri * BK), 16, off + k0 * 2, 0, 0, 0);
-    }
-    char* bs = reinterpret_cast<char*>(Bs + st * B_ST);
-#pragma unroll
-    for (int i = 0; i < B_LD; i++) {
+    } else {
+      const int k0 = kt_b * BK, j = i - A_LD;
+      char* bs = reinterpret_cast<char*>(Bs + sb * B_ST);
       if constexpr (Q8) {
-        const int ri = (wave * B_LD + i) * RPI8;
+        const int ri = (wave * B_LD + j) * RPI8;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rs, (lds_void_t*)(bs + ri * BK), 16, b_lo[0] + ri * K + k0, 0, 0, 0);
       } else {
-        const int ri = (wave * B_LD + i) * RPI;
+        const int ri = (wave * B_LD + j) * RPI;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rs, (lds_void_t*)(bs + ri * 2 * BK), 16,
                                                  b_lo[(ri / RPI) % (BK == 128 ? 4 : 2)] + ri * K * 2 + k0 * 2, 0, 0, 0);
       }
     }
   };
-
   const int fr = lane & 31, fk = lane >> 5;  // fragment row (or column) and k half
   // grouped scatter: the C row of each of this lane's fragment rows, requested now so that the
   // epilogue waits for nothing
@@ -328,26 +362,28 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
 #pragma unroll
   for (int j = 0; j < FN; j++) b_row[j] = (wn * TN + j * 32 + fr);
 
-  // fragments of step s = 2 jh + h of the tile in stage st
-  auto load_a = [&](int st, int s, f16x8 (&af)[FM]) {
-    const int c = 4 * (s >> 1) + 2 * fk + (s & 1);
-    const f16* as = As + st * A_ST;
+  // The memory instructions of one step, in the order sched_step expects: the fragments of step
+  // s = 2 jh + h of the tile in stages sa (A) and sb (W), W's first (the first MFMAs need one A
+  // fragment and all of W's), then NV DMA instructions, dma(v) the v-th. fp16 W: one fragment per
+  // step; int8 W: both steps of half jh come as one raw 16-byte chunk, read where WQ is set.
+  auto step_mem = [&](auto wq, auto nv, int sa, int sb, int s, f16x8 (&af)[FM], f16x8 (&bf)[FN], u32x4 (&bq)[FN],
+                      auto dma) {
+    const int c = 4 * (s >> 1) + 2 * fk + (s & 1), cq = 2 * (s >> 1) + fk;
+    const f16* as = As + sa * A_ST;
+    const f16* bs = Bs + sb * B_ST;
+    if constexpr (!Q8 || decltype(wq)::value) {
+#pragma unroll
+      for (int j = 0; j < FN; j++) {
+        if constexpr (Q8)
+          bq[j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(bs) + lds_off8<BK>(b_row[j], cq));
+        else
+          bf[j] = *reinterpret_cast<const f16x8*>(bs + lds_off<BK>(b_row[j], c));
+      }
+    }
 #pragma unroll
     for (int i = 0; i < FM; i++) af[i] = *reinterpret_cast<const f16x8*>(as + lds_off<BK>(a_row[i], c));
-  };
-  // fp16 W: one fragment per step
-  auto load_b = [&](int st, int s, f16x8 (&bf)[FN]) {
-    const int c = 4 * (s >> 1) + 2 * fk + (s & 1);
-    const f16* bs = Bs + st * B_ST;
 #pragma unroll
-    for (int j = 0; j < FN; j++) bf[j] = *reinterpret_cast<const f16x8*>(bs + lds_off<BK>(b_row[j], c));
-  };
-  // int8 W: both steps of half jh as one raw 16-byte chunk
-  auto load_q = [&](int st, int jh, u32x4 (&bq)[FN]) {
-    const char* bs = reinterpret_cast<const char*>(Bs + st * B_ST);
-    const int c = 2 * jh + fk;
-#pragma unroll
-    for (int j = 0; j < FN; j++) bq[j] = *reinterpret_cast<const u32x4*>(bs + lds_off8<BK>(b_row[j], c));
+    for (int v = 0; v < decltype(nv)::value; v++) dma(v);
   };
 
   f32x16 acc[FM][FN];
@@ -382,110 +418,117 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
       for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[j], af[i], acc[i][j], 0, 0, 0);
   };
 
-  // ---- prologue: S tiles in flight (past the split's last tile, its first tile again: a stage is
-  //      filled every time, so the outstanding-DMA count is the same in every iteration), the
-  //      first fragments of tile 0 in registers
+  // ---- prologue: the whole ring in flight (past the split's last tile, its first tile again: a
+  //      stage is filled every time, so the outstanding-DMA count is the same in every iteration);
+  //      the first fragments of tile 0 in registers
   auto tile_or_first = [&](int kt) { return kt < kt0 + nloc ? kt : kt0; };
 #pragma unroll
-  for (int s = 0; s < S; s++) issue(tile_or_first(kt0 + s), s);
-  wait_vmcnt<(S - 1) * L>();
+  for (int s = 0; s < SB; s++) {
+#pragma unroll
+    for (int i = 0; i < L; i++)
+      if (i >= A_LD || s < S) issue_one(i, tile_or_first(kt0 + s), s, tile_or_first(kt0 + s), s);
+  }
+  int ra = kt0, rb = kt0, rsa = 0, rsb = 0;  // the refill under way: K tiles ra / rb into stages rsa / rsb
+  wait_vmcnt<(S - 1) * A_LD + (SB - 1) * B_LD>();
   barrier_no_fence();
+  int sa = 0, sb = 0;  // the current tile's stages
   f16x8 af0[FM], af1[FM], bf0[FN], bf1[FN];
   u32x4 bq0[FN], bq1[FN];  // int8: raw chunks of the tile's first and second 32-deep half
-  load_a(0, 0, af0);
-  if constexpr (Q8) load_q(0, 0, bq0);
-  else load_b(0, 0, bf0);
+  constexpr std::true_type kWQ{};   // int8: the step that reads a half's raw chunks ...
+  constexpr std::false_type kNoQ{};  // ... and the one that does not
+  constexpr std::integral_constant<int, 0> kNoDma{};
+  auto no_dma = [](int) {};
+  step_mem(kWQ, kNoDma, 0, 0, 0, af0, bf0, bq0, no_dma);
 
   constexpr int NM = FM * FN;               // MFMAs per step
   constexpr int ND = FM + (Q8 ? 0 : FN);    // LDS reads per step (int8 W: + FN every other step)
+  // part p of the refill under way
+  auto dma_part = [&](int p) {
+    return [&, p](int v) { issue_one(part_at(p, v), ra, rsa, rb, rsb); };
+  };
+  // the tile's last fragments are in registers: the next tile has landed for every wave, and the
+  // current tile's stages are free for the next refill (its part 0 goes out in the step that
+  // follows, the other parts in the next tile's first steps)
+  auto next_tile = [&](int t) {
+    wait_lgkm0();
+    wait_vmcnt<(S - 2) * L + (SB > S ? B_LD : 0)>();
+    barrier_no_fence();
+    ra = tile_or_first(kt0 + t + S);
+    rb = tile_or_first(kt0 + t + SB);
+    rsa = sa;
+    rsb = sb;
+    sa = sa + 1 == S ? 0 : sa + 1;
+    sb = sb + 1 == SB ? 0 : sb + 1;
+  };
+  // Each depth's `tile` is one tile but the last: its steps with the parts of the refill under way
+  // (none in tile 0, whose ring the prologue has filled), and the handover to the next tile.
+  constexpr std::integral_constant<int, part_n(0)> kP0{};
   if constexpr (BK == 128) {
     // ---- 128-deep fp16 tiles (K % 128 == 0): 8 steps each, fragments one step ahead, the same
     //      k order as two consecutive 64-deep tiles (so the same sums, bit for bit)
-    for (int t = 0; t < nloc - 1; t++) {
-      const int st = t % S;
-#pragma unroll
-      for (int p = 0; p < 3; p++) {
-        load_a(st, 2 * p + 1, af1);
-        load_b(st, 2 * p + 1, bf1);
+    auto tile = [&](int t, auto refill) {
+      constexpr bool R = decltype(refill)::value && NP > 1;
+      auto pair = [&](auto part, int s) {
+        constexpr int P = decltype(part)::value;
+        constexpr std::integral_constant<int, (R ? part_n(P) : 0)> nv{};
+        step_mem(kWQ, nv, sa, sb, s, af1, bf1, bq0, dma_part(P));
         mfmas(0, af0, bf0, bq0);
-        sched_step<NM, ND>();
-        load_a(st, 2 * p + 2, af0);
-        load_b(st, 2 * p + 2, bf0);
+        sched_step<NM, ND, (R ? part_n(P) : 0)>();
+        step_mem(kWQ, kNoDma, sa, sb, s + 1, af0, bf0, bq0, no_dma);
         mfmas(0, af1, bf1, bq0);
         sched_step<NM, ND>();
-      }
-      load_a(st, 7, af1);
-      load_b(st, 7, bf1);
+      };
+      pair(std::integral_constant<int, 1>{}, 1);
+      pair(std::integral_constant<int, 2>{}, 3);
+      pair(std::integral_constant<int, 3>{}, 5);
+      step_mem(kWQ, kNoDma, sa, sb, 7, af1, bf1, bq0, no_dma);
       mfmas(0, af0, bf0, bq0);
       sched_step<NM, ND>();
-      // the tile's last fragments are in registers: free its stage, refill it, start the next tile
-      wait_lgkm0();
-      wait_vmcnt<(S - 2) * L>();
-      barrier_no_fence();
-      issue(tile_or_first(kt0 + t + S), st);
-      const int sn = (t + 1) % S;
-      load_a(sn, 0, af0);
-      load_b(sn, 0, bf0);
+      next_tile(t);
+      step_mem(kWQ, kP0, sa, sb, 0, af0, bf0, bq0, dma_part(0));
       mfmas(0, af1, bf1, bq0);
-      sched_step<NM, ND>();
-    }
-    const int st = (nloc - 1) % S;
+      sched_step<NM, ND, part_n(0)>();
+    };
+    if (nloc > 1) tile(0, std::false_type{});
+    for (int t = 1; t < nloc - 1; t++) tile(t, std::true_type{});
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-      load_a(st, 2 * p + 1, af1);
-      load_b(st, 2 * p + 1, bf1);
+      step_mem(kWQ, kNoDma, sa, sb, 2 * p + 1, af1, bf1, bq0, no_dma);
       mfmas(0, af0, bf0, bq0);
-      if (p < 3) {
-        load_a(st, 2 * p + 2, af0);
-        load_b(st, 2 * p + 2, bf0);
-      }
+      if (p < 3) step_mem(kWQ, kNoDma, sa, sb, 2 * p + 2, af0, bf0, bq0, no_dma);
       mfmas(0, af1, bf1, bq0);
     }
   } else if constexpr (BK == 64) {
-    // ---- main loop over all tiles but the last: 4 steps each, fragments one step ahead
-    for (int t = 0; t < nloc - 1; t++) {
-      const int st = t % S;
-      load_a(st, 1, af1);
-      if constexpr (!Q8) load_b(st, 1, bf1);
+    // ---- 64-deep tiles: 4 steps each, fragments one step ahead
+    auto tile = [&](int t, auto refill) {
+      constexpr bool R = decltype(refill)::value && NP > 1;
+      constexpr std::integral_constant<int, (R ? part_n(1) : 0)> p1{};
+      constexpr std::integral_constant<int, (R ? part_n(2) : 0)> p2{};
+      constexpr std::integral_constant<int, (R ? part_n(3) : 0)> p3{};
+      step_mem(kNoQ, p1, sa, sb, 1, af1, bf1, bq0, dma_part(1));
       mfmas(0, af0, bf0, bq0);
-      sched_step<NM, ND>();
-      load_a(st, 2, af0);
-      if constexpr (Q8) load_q(st, 1, bq1);
-      else load_b(st, 2, bf0);
+      sched_step<NM, ND, (R ? part_n(1) : 0)>();
+      step_mem(kWQ, p2, sa, sb, 2, af0, bf0, bq1, dma_part(2));
       mfmas(1, af1, bf1, bq0);
-      sched_step<NM, ND + (Q8 ? FN : 0)>();
-      load_a(st, 3, af1);
-      if constexpr (!Q8) load_b(st, 3, bf1);
+      sched_step<NM, ND + (Q8 ? FN : 0), (R ? part_n(2) : 0)>();
+      step_mem(kNoQ, p3, sa, sb, 3, af1, bf1, bq1, dma_part(3));
       mfmas(0, af0, bf0, bq1);
-      sched_step<NM, ND>();
-      // the tile's last fragments are in registers: free its stage, refill it, start the next tile
-      wait_lgkm0();
-      wait_vmcnt<(S - 2) * L>();
-      barrier_no_fence();
-      issue(tile_or_first(kt0 + t + S), st);
-      const int sn = (t + 1) % S;
-      load_a(sn, 0, af0);
-      if constexpr (Q8) load_q(sn, 0, bq0);
-      else load_b(sn, 0, bf0);
+      sched_step<NM, ND, (R ? part_n(3) : 0)>();
+      next_tile(t);
+      step_mem(kWQ, kP0, sa, sb, 0, af0, bf0, bq0, dma_part(0));
       mfmas(1, af1, bf1, bq1);
-      sched_step<NM, ND + (Q8 ? FN : 0)>();
-    }
+      sched_step<NM, ND + (Q8 ? FN : 0), part_n(0)>();
+    };
+    if (nloc > 1) tile(0, std::false_type{});
+    for (int t = 1; t < nloc - 1; t++) tile(t, std::true_type{});
     // ---- the last tile (its first half only when K % 64 == 32)
     {
-      const int st = (nloc - 1) % S;
-      load_a(st, 1, af1);
-      if constexpr (!Q8) load_b(st, 1, bf1);
+      step_mem(kNoQ, kNoDma, sa, sb, 1, af1, bf1, bq0, no_dma);
       mfmas(0, af0, bf0, bq0);
       mfmas(1, af1, bf1, bq0);
       if (!half_tail) {
-        load_a(st, 2, af0);
-        load_a(st, 3, af1);
-        if constexpr (Q8) {
-          load_q(st, 1, bq1);
-        } else {
-          load_b(st, 2, bf0);
-          load_b(st, 3, bf1);
-        }
+        step_mem(kWQ, kNoDma, sa, sb, 2, af0, bf0, bq1, no_dma);
+        step_mem(kNoQ, kNoDma, sa, sb, 3, af1, bf1, bq1, no_dma);
         mfmas(0, af0, bf0, bq1);
         mfmas(1, af1, bf1, bq1);
       }
@@ -493,32 +536,25 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
   } else {
     // ---- 32-deep tiles: 2 steps each, fragments one step ahead; int8 W holds both steps of a
     //      tile in one raw 16-byte chunk per fragment (bq0), the next tile's read into bqn first
-    for (int t = 0; t < nloc - 1; t++) {
-      const int st = t % S;
-      load_a(st, 1, af1);
-      if constexpr (!Q8) load_b(st, 1, bf1);
+    auto tile = [&](int t, auto refill) {
+      constexpr bool R = decltype(refill)::value && NP > 1;
+      constexpr std::integral_constant<int, (R ? part_n(1) : 0)> p1{};
+      step_mem(kNoQ, p1, sa, sb, 1, af1, bf1, bq0, dma_part(1));
       mfmas(0, af0, bf0, bq0);
-      sched_step<NM, ND>();
-      // the tile's last fragments are in registers: free its stage, refill it, start the next tile
-      wait_lgkm0();
-      wait_vmcnt<(S - 2) * L>();
-      barrier_no_fence();
-      issue(tile_or_first(kt0 + t + S), st);
-      const int sn = (t + 1) % S;
-      load_a(sn, 0, af0);
+      sched_step<NM, ND, (R ? part_n(1) : 0)>();
+      next_tile(t);
       [[maybe_unused]] u32x4 bqn[FN];
-      if constexpr (Q8) load_q(sn, 0, bqn);
-      else load_b(sn, 0, bf0);
+      step_mem(kWQ, kP0, sa, sb, 0, af0, bf0, bqn, dma_part(0));
       mfmas(1, af1, bf1, bq0);
-      sched_step<NM, ND + (Q8 ? FN : 0)>();
+      sched_step<NM, ND + (Q8 ? FN : 0), part_n(0)>();
       if constexpr (Q8) {
 #pragma unroll
         for (int j = 0; j < FN; j++) bq0[j] = bqn[j];
       }
-    }
-    const int st = (nloc - 1) % S;
-    load_a(st, 1, af1);
-    if constexpr (!Q8) load_b(st, 1, bf1);
+    };
+    if (nloc > 1) tile(0, std::false_type{});
+    for (int t = 1; t < nloc - 1; t++) tile(t, std::true_type{});
+    step_mem(kNoQ, kNoDma, sa, sb, 1, af1, bf1, bq0, no_dma);
     mfmas(0, af0, bf0, bq0);
     mfmas(1, af1, bf1, bq0);
   }
@@ -767,11 +803,19 @@ constexpr bool gemm_cfg_fits(int c, bool q8, int K) {
 // 64 rows each), so each expert's weights are streamed once; a 64-row tile split most experts into
 // two row tiles, each streaming the same weights.
 constexpr int kGrpBM = 128, kGrpBN = 128, kGrpWM = 2, kGrpWN = 2, kGrpStages = 4, kGrpBK = 64;
+// Ring stages of a config's A and W tiles. The 64-deep 256 x 256 and 256 x 192 tiles hold one more
+// stage for W than for A (in fp16, 256 x 256 fills the CU's 160 KB with it): with two stages of
+// both, each tile's DMA has less than one tile of MFMA work to land and must go out in one burst;
+// with a third W stage it is spread over the tile, A first, and W (weights, from HBM) is requested
+// two tiles ahead. int8 W rows are half as wide and leave room for one stage more of each.
+constexpr bool gemm_odd_ring(int c) { return kGemmCfgs[c].bm == 256 && kGemmCfgs[c].bn >= 192 && kGemmCfgs[c].bk == 64; }
+constexpr int gemm_sa(int c, bool q8) { return gemm_odd_ring(c) && q8 ? 3 : kGemmCfgs[c].st; }
+constexpr int gemm_sb(int c, bool q8) { return gemm_odd_ring(c) ? gemm_sa(c, q8) + 1 : kGemmCfgs[c].st; }
 // LDS of the staged epilogue: the fp16 tile with 16-byte row padding, then one C row index per row
 constexpr size_t gemm_stage_bytes(int bm, int bn) { return (size_t)bm * (bn + 8) * 2 + (size_t)bm * 4; }
 inline size_t gemm_lds_bytes(int cfg, bool q8) {
   const GemmCfg& c = kGemmCfgs[cfg];
-  const size_t ring = (size_t)c.kg * c.st * (c.bm * c.bk * 2 + c.bn * (q8 ? c.bk : 2 * c.bk));
+  const size_t ring = (size_t)c.kg * (gemm_sa(cfg, q8) * c.bm * c.bk * 2 + gemm_sb(cfg, q8) * c.bn * (q8 ? c.bk : 2 * c.bk));
   const bool staged = c.kg == 1 && c.wn == 1;  // the kernel's kStaged (grouped tiles size their own)
   return staged && gemm_stage_bytes(c.bm, c.bn) > ring ? gemm_stage_bytes(c.bm, c.bn) : ring;
 }
@@ -877,15 +921,15 @@ inline SplitkRmsnormFn splitk_rmsnorm_kernel(bool one_chunk, int splits) {
   return one_chunk ? splitk_rmsnorm_for<1>(splits) : splitk_rmsnorm_for<kNormChunks>(splits);
 }
 
-template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, int BK, int KG>
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, int BK, int KG, int SB>
 int gemm_launch(const GemmArgs& g, int cfg, int splits, hipStream_t s) {
   const size_t lds = gemm_lds_bytes(cfg, Q8);
-  const void* fn = reinterpret_cast<const void*>(&gemm_kernel<BM, BN, WM, WN, S, EPI, Q8, false, BK, KG>);
+  const void* fn = reinterpret_cast<const void*>(&gemm_kernel<BM, BN, WM, WN, S, EPI, Q8, false, BK, KG, SB>);
   const int bpc = hi_blocks_per_cu(fn, 64 * WM * WN * KG, lds);  // also lifts the dynamic-LDS limit
   if (bpc < 0) return -2;
   if (bpc == 0) HI_FAIL("gemm: tile %dx%d does not fit on a CU", BM, BN);
   const int tiles = ((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
-  hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, S, EPI, Q8, false, BK, KG>), dim3(tiles, splits),
+  hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, S, EPI, Q8, false, BK, KG, SB>), dim3(tiles, splits),
                      dim3(64 * WM * WN * KG), lds, s, g);
   HI_TRY(hipGetLastError());
   if (splits > 1 && EPI == 1 && g.norm_y) {
@@ -909,13 +953,13 @@ template <int EPI>
 int gemm_blocks_per_cu(int cfg, bool q8);
 
 #define HI_GEMM_K(i, q)                                                                                        \
-  gemm_kernel<kGemmCfgs[i].bm, kGemmCfgs[i].bn, kGemmCfgs[i].wm, kGemmCfgs[i].wn, kGemmCfgs[i].st, EPI, q, false, \
-              kGemmCfgs[i].bk, kGemmCfgs[i].kg>
+  gemm_kernel<kGemmCfgs[i].bm, kGemmCfgs[i].bn, kGemmCfgs[i].wm, kGemmCfgs[i].wn, gemm_sa(i, q), EPI, q, false,  \
+              kGemmCfgs[i].bk, kGemmCfgs[i].kg, gemm_sb(i, q)>
 #define HI_GEMM_CFG(i, q)                                                                                      \
   if constexpr (gemm_cfg_ok(i, q)) {                                                                           \
     if (cfg == i && q8 == q)                                                                                   \
-      return gemm_launch<kGemmCfgs[i].bm, kGemmCfgs[i].bn, kGemmCfgs[i].wm, kGemmCfgs[i].wn, kGemmCfgs[i].st, EPI, \
-                         q, kGemmCfgs[i].bk, kGemmCfgs[i].kg>(g, cfg, splits, s);                              \
+      return gemm_launch<kGemmCfgs[i].bm, kGemmCfgs[i].bn, kGemmCfgs[i].wm, kGemmCfgs[i].wn, gemm_sa(i, q), EPI, \
+                         q, kGemmCfgs[i].bk, kGemmCfgs[i].kg, gemm_sb(i, q)>(g, cfg, splits, s);                              \
   }
 #define HI_GEMM_OCC(i)                                                                                         \
   if constexpr (gemm_cfg_ok(i, true))                                                                          \
