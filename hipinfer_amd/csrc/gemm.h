@@ -87,16 +87,6 @@ struct GemmArgs {
 
 constexpr int kGemmBK = 64;
 constexpr int kGemmMaxGroups = 256;  // grouped mode: at most this many groups (MoE experts)
-// Wait until every LDS read of this wave has returned.
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-// Workgroup barrier without a memory fence (a fence would drain every in-flight LDS DMA); the
-// DMA completions it orders are waited for explicitly with wait_vmcnt.
-__device__ __forceinline__ void barrier_no_fence() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // Four consecutive fp16 values at p: one 8-byte access when `vec` (p 8-byte aligned), else four.
 __device__ __forceinline__ f16x4 load4(const f16* p, bool vec) {
   if (vec) return *reinterpret_cast<const f16x4*>(p);

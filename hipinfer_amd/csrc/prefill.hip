@@ -10,14 +10,20 @@
 //    SIMD let one wave's softmax run beside the other's matrix work. The wave's Q rows stay in
 //    registers as v_mfma_f32_32x32x16_f16 operands for the whole kernel;
 //  * 128-key K/V tiles of the head's cache rows go straight from global memory into LDS by buffer
-//    DMA (no register staging), two LDS stages: tile j + 1 streams in while tile j is computed,
-//    one barrier per tile. Both tiles keep the cache's row-major order with their 16-byte chunks
-//    XOR-swizzled by the key; the swizzle is applied to the DMA's per-lane source address, since
-//    a DMA instruction writes 64 consecutive 16-byte LDS slots;
+//    DMA (no register staging), two LDS stages each: K tile j + 2 and V tile j + 1 stream in while
+//    tile j is computed, one barrier per tile. Both tiles keep the cache's row-major order with their
+//    16-byte chunks XOR-swizzled by the key; the swizzle is applied to the DMA's per-lane source
+//    address, since a DMA instruction writes 64 consecutive 16-byte LDS slots;
+//  * the tiles are pipelined inside each wave: while the softmax of tile j runs on the vector units,
+//    the matrix cores work on the logits of tile j + 1 and on tile j's P.V, interleaved instruction by
+//    instruction. What bounds it: at T = 2048 after 4096 positions (Hq 32, Hkv 8, D 128) the MFMAs
+//    alone take about half of the GPU's cycles and the clock drops to 1.8 GHz under the load; 204 ->
+//    173 us (850 -> 1000 TFLOP/s) against back-to-back products, T = 1024 from 0 26.6 -> 22.1 us, 333
+//    rows after 1500 36.8 -> 27.2, D = 64 T = 2048 after 2048 76.7 -> 68;
 //  * S^T = K Q^T over the wave's 64 keys, in 32-key MFMA blocks: with the K fragment as first
 //    operand each lane ends with 16 keys per block of ONE query row (split between lanes l and
-//    l + 32), so the row max and sum of the online softmax are the lane's own values plus one
-//    exchange with lane l ^ 32;
+//    l + 32), so the row max and sum of the online softmax are the lane's own values; lanes l and
+//    l ^ 32 exchange them only where the reference max moves and at the end;
 //  * logits are scaled by log2(e) / sqrt(D) and the softmax runs in base 2 (the reference's
 //    log2-domain form, kernels.cuh:1236-1262); P is rounded to fp16 for P.V, the row sum l keeps
 //    fp32 p, as the reference does. exp2 is the hardware's v_exp_f32, whose results below 2^-126
@@ -30,10 +36,12 @@
 //    come from the row-major V tile through ds_read_tr16_b64, which transposes 4 keys x 16 d
 //    blocks within each 16-lane group; O^T keeps the lane -> query row map, so the per-row
 //    rescale by exp2(m_old - m_new) is per lane;
-//  * causal mask on absolute positions (row t at p0 + t sees keys 0..p0+t); a wave skips key
-//    halves that lie wholly above its rows' diagonal and drops the mask on halves wholly below
-//    it; cache rows past the block's last key read as zeros (the DMA's buffer range ends there);
+//  * causal mask on absolute positions (row t at p0 + t sees keys 0..p0+t): only the block's last
+//    one or two tiles (and an odd one before them) carry the mask arithmetic; cache rows past the
+//    block's last key read as zeros (the DMA's buffer range ends there);
 //  * blocks run the longest query tiles (the most keys) first, across all heads.
+#include <type_traits>
+
 #include "hi_common.h"
 
 namespace {
@@ -61,16 +69,17 @@ __device__ __forceinline__ int v_swz(int r) {
   return ((2 * a) ^ (4 * a)) & (D / 8 - 1);
 }
 
-template <int D>
-struct FpStage {
-  u32x4 k[kFpBKV * D / 8];
-  u32x4 v[kFpBKV * D / 8];
-};
-// The O^T accumulators the second wave of each row group hands to the first at the end (in the
-// stages' LDS).
+// LDS of one block: two stages of K tiles and two of V tiles while the keys stream, then in the same
+// bytes the O^T accumulators the second wave of each row group hands to the first; last, the second
+// waves' m and l. It is dynamic LDS: reads of a __shared__ array that a DMA instruction also writes
+// made the compiler wait for every DMA in flight (s_waitcnt vmcnt(0)) before the first of them, right
+// after the next tile's DMA had been issued, so that no tile streamed in while another was computed.
 template <int D, int RG>
-struct FpMerge {
-  f32x16 o[RG][D / 32][64];
+struct FpSmem {
+  static constexpr int kTile = kFpBKV * D / 8;                // 16-byte chunks of one K or V tile
+  static constexpr int kMl = 2 * kFpStages * kTile;           // chunk index of m and l
+  static constexpr size_t kBytes = kMl * 16 + 2 * RG * 64 * 4;
+  static_assert(RG * (D / 32) * 64 * 64 <= kMl * 16, "merge fits the stages");
 };
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -85,7 +94,7 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rs, void* lds, 
 }
 // ds_read_tr16_b64 at LDS address p: within each 16-lane group, lane i receives element i % 4 of
 // the 4 halves lane 4 e + i / 4 addresses, as its element e.
-__device__ __forceinline__ f16x4 lds_read_tr16(const f16* p) {
+__device__ __forceinline__ f16x4 lds_read_tr16(const f16* __restrict__ p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)p));
 #else
@@ -102,12 +111,17 @@ __global__ void __launch_bounds__(128 * RG)
   constexpr int CPR = D / 8;                   // 16-byte chunks per key row
   constexpr int IPW = kFpBKV * CPR / 64 / NW;  // DMA instructions per wave per tile and operand
   constexpr int DT = D / 32;                   // 32-row output tiles of O^T
+  constexpr int NQ = D / 16;                   // MFMAs of one 32-key block's logits
   static_assert(IPW * 64 * NW == kFpBKV * CPR, "tile DMA split");
-  static_assert(sizeof(FpMerge<D, RG>) <= sizeof(FpStage<D>) * kFpStages, "merge fits the stages");
-  __shared__ FpStage<D> sm[kFpStages];
-  __shared__ float ml[2][RG][64];  // the second waves' m and l
+  static_assert(kFpStages == 2 && kFpKPW == 64, "the tile body is written for two stages and two key blocks");
+  using Sm = FpSmem<D, RG>;
+  extern __shared__ u32x4 fp_smem[];
+  u32x4* const ks_ = fp_smem;                                // [2][kTile]: K stages
+  u32x4* const vs_ = fp_smem + kFpStages * Sm::kTile;        // [2][kTile]: V stages
+  f32x16* const mo = reinterpret_cast<f32x16*>(fp_smem);     // [RG][DT][64]: the merge
+  float* const ml = reinterpret_cast<float*>(fp_smem + Sm::kMl);  // [2][RG][64]: the second waves' m and l
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = wave % RG, kh = wave / RG;     // row group, key half
   const int fr = lane & 31, fk = lane >> 5;
   // grid (Hq, query tiles), dispatched x first: all heads' longest query tile first; block x runs
@@ -118,12 +132,23 @@ __global__ void __launch_bounds__(128 * RG)
   const int qi = qw + fr;                       // this lane's query row
   const int qpos = p0 + qi;
   const int kv_end = p0 + min(q0 + BQ, T);      // keys any row of the block can see
+  const int nt = (kv_end + kFpBKV - 1) / kFpBKV;  // key tiles; the first n_full hold no masked key
+  const int n_full = (p0 + q0 + 1) / kFpBKV;
+
+  // this lane's Q fragments: row qi, d = 16 ks + 8 fk + 0..7 (zero past T)
+  f16x8 qf[NQ];
+#pragma unroll
+  for (int ks = 0; ks < NQ; ks++) {
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (qi < T) v = *reinterpret_cast<const u32x4*>(q + (int64_t)qi * ldq + h * D + 16 * ks + 8 * fk);
+    qf[ks] = __builtin_bit_cast(f16x8, v);
+  }
+
   // the head's cache rows 0..kv_end-1: loads past them return zeros
   const __amdgpu_buffer_rsrc_t k_rs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<f16*>(kc + (int64_t)hk * max_seq * D), (short)0, kv_end * D * 2, 0x00020000);
   const __amdgpu_buffer_rsrc_t v_rs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<f16*>(vc + (int64_t)hk * max_seq * D), (short)0, kv_end * D * 2, 0x00020000);
-
   // DMA instruction i of this wave fills slots (wave IPW + i) * 64 + lane of a tile: slot s holds
   // key s / CPR, physical chunk s % CPR, i.e. logical chunk (s % CPR) ^ swz(key)
   int koff[IPW], voff[IPW];
@@ -133,23 +158,17 @@ __global__ void __launch_bounds__(128 * RG)
     koff[i] = (r * D + 8 * (p ^ k_swz<D>(r))) * 2;
     voff[i] = (r * D + 8 * (p ^ v_swz<D>(r))) * 2;
   }
-  auto issue = [&](int j0, int st) {
-#pragma unroll
-    for (int i = 0; i < IPW; i++) {
-      lds_dma16(k_rs, &sm[st].k[(wave * IPW + i) * 64], koff[i] + j0 * D * 2);
-      lds_dma16(v_rs, &sm[st].v[(wave * IPW + i) * 64], voff[i] + j0 * D * 2);
-    }
+  // issue instruction i of the next K (V) tile into stage st; koff / voff then point at the one after
+  auto issue_k = [&](int i, int st) {
+    lds_dma16(k_rs, ks_ + st * Sm::kTile + (wave * IPW + i) * 64, koff[i]);
+    koff[i] += kFpBKV * D * 2;
+    asm volatile("" : "+v"(koff[i]));  // one running offset, not a base and an induction variable
   };
-  issue(0, 0);
-
-  // this lane's Q fragments: row qi, d = 16 ks + 8 fk + 0..7 (zero past T)
-  f16x8 qf[D / 16];
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ks++) {
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (qi < T) v = *reinterpret_cast<const u32x4*>(q + (int64_t)qi * ldq + h * D + 16 * ks + 8 * fk);
-    qf[ks] = __builtin_bit_cast(f16x8, v);
-  }
+  auto issue_v = [&](int i, int st) {
+    lds_dma16(v_rs, vs_ + st * Sm::kTile + (wave * IPW + i) * 64, voff[i]);
+    voff[i] += kFpBKV * D * 2;
+    asm volatile("" : "+v"(voff[i]));
+  };
 
   // transpose reads of V: lane j of each 16-lane group g reads 4 d of key 4 (g / 2) + j / 4 (+ the
   // step's key base), d = 16 (g % 2) + 4 (j % 4) (+ the output tile's d base); the group's lane i
@@ -157,8 +176,10 @@ __global__ void __launch_bounds__(128 * RG)
   // term is the lane's own.
   const int vr = 4 * fk + ((lane & 15) >> 2);                  // key within a 16-key step
   const int vc0 = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);   // logical chunk within a 32-d tile
-  const int vsw = v_swz<D>(vr), vh = 4 * (lane & 1);           // swizzle term, half within the chunk
-  constexpr int KT = kFpKPW / 32;                              // 32-key blocks per wave per tile
+  const f16* vb[DT];                                           // the lane's first read of each output tile
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+    vb[dt] = reinterpret_cast<const f16*>(vs_) + (kFpKPW * kh + vr) * D + 8 * ((4 * dt + vc0) ^ v_swz<D>(vr)) + 4 * (lane & 1);
   const int kr = kFpKPW * kh + fr;                             // K row of this lane's first fragments
   const int ksw = k_swz<D>(kr);                                // the same for every block (kr % 16)
   const int xaddr = (lane ^ 32) << 2;                          // lane l ^ 32, for ds_bpermute
@@ -166,6 +187,8 @@ __global__ void __launch_bounds__(128 * RG)
     return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(xaddr, __builtin_bit_cast(int, v)));
   };
 
+  // m_i: the row's reference max (the same in lanes l and l ^ 32); l_i: this lane's share of the
+  // row's sum (its own keys; the two lanes' shares are added at the end)
   float m_i = -__builtin_huge_valf(), l_i = 0.f;
   f32x16 o[DT];
 #pragma unroll
@@ -173,105 +196,200 @@ __global__ void __launch_bounds__(128 * RG)
 #pragma unroll
     for (int e = 0; e < 16; e++) o[dt][e] = 0.f;
 
-  int st = 0;
-  for (int j0 = 0; j0 < kv_end; j0 += kFpBKV, st ^= 1) {
-    wait_vmcnt<0>();  // this wave's share of tile j0 is in LDS
-    __syncthreads();  // every share is, and every wave is done with the other stage
-    if (j0 + kFpBKV < kv_end) issue(j0 + kFpBKV, st ^ 1);
-    const int k0 = j0 + kFpKPW * kh;                // this wave's first key
-    if (k0 > p0 + qw + 31 || k0 >= kv_end) continue;  // every key of the half is masked for every row
-    const bool full = k0 + kFpKPW - 1 <= p0 + qw && k0 + kFpKPW <= kv_end;  // no key of the half is masked
-    const u32x4* ks_ = sm[st].k;
-    const f16* vs_ = reinterpret_cast<const f16*>(sm[st].v);
-
-    // ---- S^T = K Q^T over the wave's keys, 32 per block kt; lane (row fr, half fk) gets keys
-    //      32 kt + 8 g + 4 fk + e
-    f32x16 s[KT];
+  // S^T = K Q^T over 32-key block kt of the wave's keys in K stage st; lane (row fr, half fk) gets
+  // keys 32 kt + 8 g + 4 fk + e
+  auto logits = [&](int st, int kt, f32x16& s) {
+    f32x16 a;
 #pragma unroll
-    for (int kt = 0; kt < KT; kt++) {
+    for (int e = 0; e < 16; e++) a[e] = 0.f;
 #pragma unroll
-      for (int e = 0; e < 16; e++) s[kt][e] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < D / 16; ks++) {
-        const f16x8 kf = __builtin_bit_cast(f16x8, ks_[(kr + 32 * kt) * CPR + ((2 * ks + fk) ^ ksw)]);
-        s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[ks], s[kt], 0, 0, 0);
-      }
+    for (int ks = 0; ks < NQ; ks++) {
+      const f16x8 kf = __builtin_bit_cast(f16x8, ks_[st * Sm::kTile + (kr + 32 * kt) * CPR + ((2 * ks + fk) ^ ksw)]);
+      a = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[ks], a, 0, 0, 0);
     }
-    // ---- online softmax of row qi over these keys (base 2). The row's reference max m_i moves
-    //      only when the tile's scaled max exceeds it by more than 2^8, so p = exp2(c s - m_i) stays
-    //      at most 256 (exact range for fp16 P and fp32 sums) and O is rescaled only then; the
-    //      max of the raw logits is scaled once (c > 0 keeps the order) and c s - m_i is one fma
-    float mx = -__builtin_huge_valf();
-    if (full) {
+    s = a;
+  };
+  // the V^T fragments of block kt (V stage st): of step ss, lane half fk holds keys 32 kt + 16 ss +
+  // 4 fk + 0..3 and 32 kt + 16 ss + 8 + 4 fk + 0..3 of the wave's keys, as P's registers do
+  auto load_v = [&](int st, int kt, f16x8 (&vf)[2][DT]) {
 #pragma unroll
-      for (int kt = 0; kt < KT; kt++)
+    for (int ss = 0; ss < 2; ss++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) mx = fmaxf(mx, s[kt][e]);
-    } else {
+      for (int dt = 0; dt < DT; dt++) {
+        const f16* pa = vb[dt] + st * (Sm::kTile * 8) + (32 * kt + 16 * ss) * D;
+        const f16x4 fa = lds_read_tr16(pa), fb = lds_read_tr16(pa + 8 * D);  // key + 8: same swizzle term
+        vf[ss][dt] = f16x8{fa[0], fa[1], fa[2], fa[3], fb[0], fb[1], fb[2], fb[3]};
+      }
+  };
+  // O^T += V^T P^T of one 32-key block
+  auto pv = [&](const f16x8 (&vf)[2][DT], const f16x8 (&pf)[2]) {
 #pragma unroll
-      for (int kt = 0; kt < KT; kt++)
+    for (int ss = 0; ss < 2; ss++)
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[ss][dt], pf[ss], o[dt], 0, 0, 0);
+  };
+  // p = exp2(c s - m) of one block, its sum into l_i, fp16 p in P.V operand order
+  auto softmax = [&](const f32x16& s, float m_use, f16x8 (&pf)[2]) {
+    float sum0 = 0.f, sum1 = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], scale_log2, -m_use));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e + 1], scale_log2, -m_use));
+      sum0 += p;
+      sum1 += p1;
+      pf[e >> 3][e & 7] = (f16)p;
+      pf[e >> 3][(e & 7) + 1] = (f16)p1;
+    }
+    l_i += sum0 + sum1;
+  };
+
+  // One key tile t (stage t & 1, given as a constant in the main loop): the softmax and P.V of its
+  // logits sc, with the logits of tile t + 1 into sn in between. A wave issues in order, so the
+  // MFMAs of one product are interleaved with the vector work of the other tile's softmax by
+  // scheduling groups; otherwise each product's MFMAs run back to back, then the softmax with the
+  // matrix cores idle (both waves of a SIMD leave the tile's barrier together). The P.V of the
+  // tile's second block (pl, its V fragments vl read before the next barrier) runs after that
+  // barrier: matrix work that needs no LDS while the first K fragments are on their way.
+  f16x8 pl[2], vl[2][DT];
+#pragma unroll
+  for (int ss = 0; ss < 2; ss++) {
+    pl[ss] = f16x8{};
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) vl[ss][dt] = f16x8{};
+  }
+  auto tile = [&](auto stc, auto maskc, auto nextc, int t, f32x16 (&sc)[2], f32x16 (&sn)[2]) {
+    constexpr bool MASK = decltype(maskc)::value;  // the tile holds keys past some row's diagonal
+    constexpr bool NEXT = decltype(nextc)::value;  // there is a tile t + 1
+    const int st = stc;
+    wait_lgkm0();
+    wait_vmcnt<0>();     // this wave's shares of K tile t + 1 and V tile t are in LDS
+    barrier_no_fence();  // every share is, and every wave is done with K tile t and V tile t - 1
+    const int k0 = t * kFpBKV + kFpKPW * kh;  // this wave's first key
+    if constexpr (MASK) {
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++)
 #pragma unroll
         for (int e = 0; e < 16; e++) {
           const int kp = k0 + 32 * kt + 8 * (e >> 2) + 4 * fk + (e & 3);
-          const float v = (kp <= qpos && kp < kv_end) ? s[kt][e] : -__builtin_huge_valf();
-          s[kt][e] = v;
-          mx = fmaxf(mx, v);
+          if (kp > qpos) sc[kt][e] = -__builtin_huge_valf();
         }
     }
-    mx = fmaxf(mx, xor32(mx)) * scale_log2;
-    const bool move = mx > m_i + kFpMaxLag;  // m_i = -inf: moves to the first finite max
-    const float alpha = move ? __builtin_amdgcn_exp2f(m_i - mx) : 1.f;
-    if (move) m_i = mx;
-    // m_i is -inf only for a row that has seen no key yet (a row past T, or one whose first key
-    // lies in the other half): every logit is then -inf and every p 0
-    const float m_use = m_i == -__builtin_huge_valf() ? 0.f : m_i;
-    float sum = 0.f;
-    f16x8 pf[KT][2];
+    // the row's reference max m_i moves only when the tile's scaled max exceeds it by more than 2^8,
+    // so p = exp2(c s - m_i) stays at most 256 (exact range for fp16 P and fp32 sums) and O is
+    // rescaled only then; lanes l and l ^ 32 then agree on the new one. The max of the raw logits is
+    // scaled once (c > 0 keeps the order) and c s - m_i is one fma
+    float mx = -__builtin_huge_valf();
+    pv(vl, pl);
+    if constexpr (NEXT) {
+      logits(st ^ 1, 0, sn[0]);
 #pragma unroll
-    for (int kt = 0; kt < KT; kt++)
+      for (int i = 0; i < IPW; i++) issue_k(i, st);
 #pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][e], scale_log2, -m_use));
-        sum += p;
-        pf[kt][e >> 3][e & 7] = (f16)p;
+      for (int i = 0; i < IPW; i++) issue_v(i, st ^ 1);
+    }
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) mx = fmaxf(mx, sc[kt][e]);
+    constexpr int kMaskOps = MASK ? 8 : 0;  // more vector work per MFMA
+#pragma unroll
+    for (int i = 0; i < 2 * DT; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (the last block's P.V)
+      if (NEXT && i >= 1 && i < 5) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS reads
+      __builtin_amdgcn_sched_group_barrier(0x002, 2 + kMaskOps, 0);  // VALU (the max)
+    }
+    if constexpr (NEXT) {
+#pragma unroll
+      for (int i = 0; i < NQ; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (logits)
+        if (i < NQ - 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 2 * IPW / NQ, 0);  // DMA
       }
-    sum += xor32(sum);
-    l_i = l_i * alpha + sum;
-    if (__any(move)) {
+    }
+    if (__any(mx * scale_log2 > m_i + kFpMaxLag)) {  // m_i = -inf: moves to the first finite max
+      mx = fmaxf(mx, xor32(mx)) * scale_log2;
+      const bool move = mx > m_i + kFpMaxLag;
+      const float alpha = move ? __builtin_amdgcn_exp2f(m_i - mx) : 1.f;
+      if (move) m_i = mx;
+      l_i *= alpha;
 #pragma unroll
       for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int e = 0; e < 16; e++) o[dt][e] *= alpha;
     }
-    // ---- O^T += V^T P^T; step ss of block kt: lane half fk holds keys 32 kt + 16 ss + 4 fk + 0..3
-    //      and 32 kt + 16 ss + 8 + 4 fk + 0..3 of the wave's keys, in P's registers and in the V^T
-    //      reads alike
+    // m_i is -inf only for a row that has seen no key yet (one whose first key lies in the other
+    // half): every logit is then -inf and every p 0
+    const float m_use = m_i == -__builtin_huge_valf() ? 0.f : m_i;
+    f16x8 pf[2], vf[2][DT];
+    if constexpr (NEXT) logits(st ^ 1, 1, sn[1]);
+    softmax(sc[0], m_use, pf);
+    load_v(st, 0, vf);
+    pv(vf, pf);
+    softmax(sc[1], m_use, pl);
+    load_v(st, 1, vl);
+    if constexpr (NEXT) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);               // LDS reads run three MFMAs ahead
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++)
+      for (int i = 0; i < NQ; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (logits)
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (i >= NQ - 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 56 / NQ, 0);       // VALU (softmax of block 0)
+      }
 #pragma unroll
-      for (int kt = 0; kt < KT; kt++)
+      for (int i = 0; i < 2 * DT; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (P.V of block 0)
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 56 / (2 * DT), 0); // VALU (softmax of block 1)
+      }
+    }
+  };
+
+  // ---- prologue: K tiles 0 and 1 and V tile 0 in flight, the logits of tile 0
 #pragma unroll
-        for (int ss = 0; ss < 2; ss++) {
-          const int key = kFpKPW * kh + 32 * kt + 16 * ss + vr;
-          const f16* pa = vs_ + key * D + 8 * ((4 * dt + vc0) ^ vsw) + vh;
-          const f16x4 fa = lds_read_tr16(pa), fb = lds_read_tr16(pa + 8 * D);  // key + 8: same swizzle term
-          const f16x8 vf = {fa[0], fa[1], fa[2], fa[3], fb[0], fb[1], fb[2], fb[3]};
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[kt][ss], o[dt], 0, 0, 0);
-        }
+  for (int i = 0; i < IPW; i++) issue_k(i, 0);
+#pragma unroll
+  for (int i = 0; i < IPW; i++) {
+    issue_v(i, 0);
+    issue_k(i, 1);
   }
+  wait_vmcnt<2 * IPW>();
+  barrier_no_fence();
+  f32x16 sa[2], sb[2];
+  logits(0, 0, sa[0]);
+  logits(0, 1, sa[1]);
+  constexpr std::integral_constant<int, 0> kEven{};
+  constexpr std::integral_constant<int, 1> kOdd{};
+  int t = 0;
+  const std::true_type yes{};
+  const std::false_type no{};
+  for (; t + 2 <= n_full && t + 2 < nt; t += 2) {
+    tile(kEven, no, yes, t, sa, sb);
+    tile(kOdd, no, yes, t + 1, sb, sa);
+  }
+  for (; t + 1 < nt; t++) {  // an odd full tile, the first of two tiles on the diagonal
+    tile(t & 1, yes, yes, t, sa, sb);
+    sa[0] = sb[0];
+    sa[1] = sb[1];
+  }
+  tile(t & 1, yes, no, t, sa, sb);
+
+  pv(vl, pl);
 
   // ---- merge the two key halves of each row group: the second wave hands (m, l, O) over
-  __syncthreads();  // every wave is done with the stages (no DMA is in flight after the last tile)
-  FpMerge<D, RG>& mg = *reinterpret_cast<FpMerge<D, RG>*>(sm);
+  wait_vmcnt<0>();
+  __syncthreads();  // every wave is done with the stages, and no DMA is in flight
+  l_i += xor32(l_i);
   if (kh == 1) {
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++) mg.o[rg][dt][lane] = o[dt];
-    ml[0][rg][lane] = m_i;
-    ml[1][rg][lane] = l_i;
+    for (int dt = 0; dt < DT; dt++) mo[(rg * DT + dt) * 64 + lane] = o[dt];
+    ml[rg * 64 + lane] = m_i;
+    ml[(RG + rg) * 64 + lane] = l_i;
   }
   __syncthreads();
   if (kh == 1 || qi >= T) return;
-  const float m1 = ml[0][rg][lane], l1 = ml[1][rg][lane];
+  const float m1 = ml[rg * 64 + lane], l1 = ml[(RG + rg) * 64 + lane];
   const float m = fmaxf(m_i, m1);  // finite: key 0 is visible to every row
   const float a0 = __builtin_amdgcn_exp2f(m_i - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
   const float l = l_i * a0 + l1 * a1;
@@ -280,7 +398,7 @@ __global__ void __launch_bounds__(128 * RG)
   f16* orow = out + (int64_t)qi * ldo + h * D;
 #pragma unroll
   for (int dt = 0; dt < DT; dt++) {
-    const f32x16 o1 = mg.o[rg][dt][lane];
+    const f32x16 o1 = mo[(rg * DT + dt) * 64 + lane];
 #pragma unroll
     for (int g = 0; g < 4; g++) {
       f16x4 v;
@@ -379,12 +497,13 @@ int flash_prefill(const void* q, int ldq, const void* kc, const void* vc, int ma
   if ((T + kFpBQ - 1) / kFpBQ > 65535) HI_FAIL("%s: T=%d exceeds %d query rows", who, T, 65535 * kFpBQ);
   const dim3 grid(Hq, (T + kFpBQ - 1) / kFpBQ);
   const hipStream_t s = (hipStream_t)stream;
-  if (D == 128)
-    hipLaunchKernelGGL((flash_prefill_kernel<128, kFpRG>), grid, dim3(128 * kFpRG), 0, s, (const f16*)q, (int64_t)ldq,
-                       (const f16*)kc, (const f16*)vc, max_seq, (f16*)out, (int64_t)ldo, T, p0, Hq, Hkv, scale_log2, lse);
-  else
-    hipLaunchKernelGGL((flash_prefill_kernel<64, kFpRG>), grid, dim3(128 * kFpRG), 0, s, (const f16*)q, (int64_t)ldq,
-                       (const f16*)kc, (const f16*)vc, max_seq, (f16*)out, (int64_t)ldo, T, p0, Hq, Hkv, scale_log2, lse);
+  const auto kern = D == 128 ? flash_prefill_kernel<128, kFpRG> : flash_prefill_kernel<64, kFpRG>;
+  const size_t lds = D == 128 ? FpSmem<128, kFpRG>::kBytes : FpSmem<64, kFpRG>::kBytes;
+  const int bpc = hi_blocks_per_cu(reinterpret_cast<const void*>(kern), 128 * kFpRG, lds);  // lifts the LDS limit
+  if (bpc < 0) return -2;
+  if (bpc == 0) HI_FAIL("%s: the kernel does not fit on a CU", who);
+  hipLaunchKernelGGL(kern, grid, dim3(128 * kFpRG), lds, s, (const f16*)q, (int64_t)ldq, (const f16*)kc, (const f16*)vc,
+                     max_seq, (f16*)out, (int64_t)ldo, T, p0, Hq, Hkv, scale_log2, lse);
   HI_TRY(hipGetLastError());
   return 0;
 }

@@ -112,6 +112,24 @@ def test_flash_prefill(hi, O, D, Hq, Hkv):
               2e-3, 1e-2)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("p0", [0, 1, 126, 127, 128, 129, 254, 255, 256, 383, 384, 511])
+def test_flash_prefill_tile_edges(hi, O, D, p0):
+    """Every count and parity of unmasked 128-key tiles before the diagonal (none to four), one or two
+    masked tiles after them, a last tile of a single key, and query blocks of 1, 127, 128 and 129
+    rows. Output and lse against the oracle."""
+    r = rng(1270 + D + p0)
+    Hq, Hkv, S = 2, 1, 704
+    kc = r.standard_normal((Hkv, S, D)).astype(np.float16)
+    vc = r.standard_normal((Hkv, S, D)).astype(np.float16)
+    for T in [1, 2, 127, 128, 129]:
+        q = r.standard_normal((T, Hq * D)).astype(np.float16)
+        out, lse = hi.flash_prefill_lse(cuda(q), cuda(kc), cuda(vc), T, p0, Hq, Hkv)
+        ref, ref_lse = O.flash_prefill(q, kc, vc, T, p0, Hq, Hkv, lse=True)
+        check(f"flash prefill D={D} T={T} p0={p0}", host(out), ref, 2e-3, 1e-2)
+        check(f"flash prefill lse D={D} T={T} p0={p0}", host(lse), ref_lse, 1e-4, 1e-5)
+
+
 def test_flash_prefill_fused_qkv_rows_and_lse(hi, O):
     """q read in place from the rows of a fused qkv buffer (ldq = (Hq + 2 Hkv) D), output into a
     padded buffer (ldo > Hq D, the padding untouched), lse against the oracle's."""
