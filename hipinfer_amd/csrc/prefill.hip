@@ -4,7 +4,7 @@
 // hi_flash_prefill_lse; api.cu:594-623, kernels.cuh:1160-1329, ctypes hipinfer.py:171-202).
 //
 // Flash prefill for gfx950 (D = 64 or 128):
-//  * block = 32 RG query rows of one query head and 2 RG waves: the waves of row group g (g and
+//  * block = 32 RG query rows (RG 4, or 2 for small grids) of one query head and 2 RG waves: the waves of row group g (g and
 //    g + RG) share its 32 rows and split every 128-key tile, keys 0..63 and 64..127, each with its
 //    own online-softmax state; the pair merges (m, l, O) through LDS at the end. Two waves per
 //    SIMD let one wave's softmax run beside the other's matrix work. The wave's Q rows stay in
@@ -46,8 +46,7 @@
 
 namespace {
 
-constexpr int kFpRG = 4;              // 32-row groups per block (2 waves each)
-constexpr int kFpBQ = 32 * kFpRG;     // query rows per block
+constexpr int kFpRG = 4;              // 32-row groups per block (2 waves each); 2 for small grids
 constexpr int kFpKPW = 64;            // keys per wave per tile (32-key MFMA blocks of the wave's half)
 constexpr int kFpBKV = 2 * kFpKPW;    // keys per tile
 constexpr int kFpStages = 2;          // LDS stages of K/V tiles
@@ -278,14 +277,48 @@ __global__ void __launch_bounds__(128 * RG)
     // so p = exp2(c s - m_i) stays at most 256 (exact range for fp16 P and fp32 sums) and O is
     // rescaled only then; lanes l and l ^ 32 then agree on the new one. The max of the raw logits is
     // scaled once (c > 0 keeps the order) and c s - m_i is one fma
+    // The MFMAs of this tile up to its first P.V, in slots: the last block's P.V, then (NEXT) the
+    // logits of tile t + 1. The 2 IPW DMA instructions of K tile t + 2 and V tile t + 1 go out over the
+    // slots of the first logits block; with 4 waves, each issuing twice as many and without a second
+    // wave on its SIMD to fill its stalls, over all of them (64 rows after 2000 positions 26.1 ->
+    // 22.6 us, 512 after 2048 36.0 -> 32.7; 8 waves: no gain, 2 % slower at T = 2048 after 4096).
+    constexpr int ND = 2 * IPW, LA = 3;  // DMA instructions, LDS reads ahead of their MFMA
+    constexpr int S0 = RG == 2 ? 0 : 2 * DT, NS = RG == 2 ? 2 * DT + 2 * NQ : NQ;
+    auto dma_here = [](int m) constexpr {  // DMA instructions that go before slot m
+      int n = 0;
+      for (int j = 0; j < ND; j++) n += S0 + j * NS / ND == m;
+      return n;
+    };
+    constexpr int kDma = (ND + NS - 1) / NS;  // at most this many before one slot
+    auto dma = [&](int m) {
+#pragma unroll
+      for (int j = 0; j < ND; j++)
+        if (S0 + j * NS / ND == m) j < IPW ? issue_k(j, st) : issue_v(j - IPW, st ^ 1);
+    };
+    auto load_k = [&](int kt, int ks) {
+      return __builtin_bit_cast(f16x8, ks_[(st ^ 1) * Sm::kTile + (kr + 32 * kt) * CPR + ((2 * ks + fk) ^ ksw)]);
+    };
     float mx = -__builtin_huge_valf();
-    pv(vl, pl);
+    f16x8 kf[NQ];
+    f32x16 a0;
+#pragma unroll
+    for (int e = 0; e < 16; e++) a0[e] = 0.f;
+#pragma unroll
+    for (int m = 0; m < 2 * DT; m++) {
+      if constexpr (NEXT) {
+        dma(m);
+        if (m >= 2 * DT - LA) kf[m - (2 * DT - LA)] = load_k(0, m - (2 * DT - LA));
+      }
+      o[m % DT] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[m / DT][m % DT], pl[m / DT], o[m % DT], 0, 0, 0);
+    }
     if constexpr (NEXT) {
-      logits(st ^ 1, 0, sn[0]);
 #pragma unroll
-      for (int i = 0; i < IPW; i++) issue_k(i, st);
-#pragma unroll
-      for (int i = 0; i < IPW; i++) issue_v(i, st ^ 1);
+      for (int ks = 0; ks < NQ; ks++) {
+        dma(2 * DT + ks);
+        if (ks + LA < NQ) kf[ks + LA] = load_k(0, ks + LA);
+        a0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], a0, 0, 0, 0);
+      }
+      sn[0] = a0;
     }
 #pragma unroll
     for (int kt = 0; kt < 2; kt++)
@@ -293,18 +326,19 @@ __global__ void __launch_bounds__(128 * RG)
       for (int e = 0; e < 16; e++) mx = fmaxf(mx, sc[kt][e]);
     constexpr int kMaskOps = MASK ? 8 : 0;  // more vector work per MFMA
 #pragma unroll
-    for (int i = 0; i < 2 * DT; i++) {
+    for (int m = 0; m < 2 * DT; m++) {
+      if (NEXT && dma_here(m)) __builtin_amdgcn_sched_group_barrier(0x020, kDma, 0);  // DMA
+      if (NEXT && m >= 2 * DT - LA) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (the last block's P.V)
-      if (NEXT && i >= 1 && i < 5) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS reads
       __builtin_amdgcn_sched_group_barrier(0x002, 2 + kMaskOps, 0);  // VALU (the max)
     }
     if constexpr (NEXT) {
 #pragma unroll
-      for (int i = 0; i < NQ; i++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (logits)
-        if (i < NQ - 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      for (int ks = 0; ks < NQ; ks++) {
+        if (dma_here(2 * DT + ks)) __builtin_amdgcn_sched_group_barrier(0x020, kDma, 0);
+        if (ks + LA < NQ) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);           // MFMA (logits)
         __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x020, 2 * IPW / NQ, 0);  // DMA
       }
     }
     if (__any(mx * scale_log2 > m_i + kFpMaxLag)) {  // m_i = -inf: moves to the first finite max
@@ -322,19 +356,33 @@ __global__ void __launch_bounds__(128 * RG)
     // half): every logit is then -inf and every p 0
     const float m_use = m_i == -__builtin_huge_valf() ? 0.f : m_i;
     f16x8 pf[2], vf[2][DT];
-    if constexpr (NEXT) logits(st ^ 1, 1, sn[1]);
+    if constexpr (NEXT) {
+      f32x16 a1;
+#pragma unroll
+      for (int e = 0; e < 16; e++) a1[e] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < LA; ks++) kf[ks] = load_k(1, ks);
+#pragma unroll
+      for (int ks = 0; ks < NQ; ks++) {
+        dma(2 * DT + NQ + ks);
+        if (ks + LA < NQ) kf[ks + LA] = load_k(1, ks + LA);
+        a1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], a1, 0, 0, 0);
+      }
+      sn[1] = a1;
+    }
     softmax(sc[0], m_use, pf);
     load_v(st, 0, vf);
     pv(vf, pf);
     softmax(sc[1], m_use, pl);
     load_v(st, 1, vl);
     if constexpr (NEXT) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);               // LDS reads run three MFMAs ahead
+      __builtin_amdgcn_sched_group_barrier(0x100, LA, 0);
 #pragma unroll
-      for (int i = 0; i < NQ; i++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (logits)
+      for (int ks = 0; ks < NQ; ks++) {
+        if (dma_here(2 * DT + NQ + ks)) __builtin_amdgcn_sched_group_barrier(0x020, kDma, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (i >= NQ - 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (ks + LA >= NQ) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA (logits)
         __builtin_amdgcn_sched_group_barrier(0x002, 56 / NQ, 0);       // VALU (softmax of block 0)
       }
 #pragma unroll
@@ -494,16 +542,29 @@ int flash_prefill(const void* q, int ldq, const void* kc, const void* vc, int ma
   if (!aligned(kc, 16) || !aligned(vc, 16)) HI_FAIL("%s: kc / vc must be 16-byte aligned", who);
   if (!aligned(out, 8) || ldo % 4 || ldo < Hq * D) HI_FAIL("%s: out must be 8-byte aligned, ldo %% 4 == 0, ldo >= Hq*D", who);
   const float scale_log2 = 1.4426950408889634f / sqrtf((float)D);
-  if ((T + kFpBQ - 1) / kFpBQ > 65535) HI_FAIL("%s: T=%d exceeds %d query rows", who, T, 65535 * kFpBQ);
-  const dim3 grid(Hq, (T + kFpBQ - 1) / kFpBQ);
+  const HiDevice* d = hi_device();
+  if (!d) return -2;
+  // Query rows per block: 128, or 64 while that grid is still resident at once. A CU takes a key tile
+  // for 64 rows only 10-25 % faster than for 128, but the longest query tile is half as tall and a
+  // small grid reaches twice the CUs: T = 512 from 0 (Hq 32, D 128) 14.4 -> 11.1 us, 64 rows after
+  // 2000 28.4 -> 22.6, 777 rows of 12 heads 16.6 -> 12.7; past one round it loses (640 rows after 2048
+  // 39.8 -> 48.9). At D = 64 two such blocks share a CU: that pays while most tiles are short of
+  // the diagonal (777 rows from 0 12.3 -> 10.2 us), not after a long prefix (960 after 2048 34.5 -> 35.3).
+  const int slots = D == 64 && p0 < T ? 2 * d->cus : d->cus;
+  const bool small = (int64_t)Hq * ((T + 63) / 64) <= slots;
+  const int rg = small ? 2 : kFpRG, bq = 32 * rg;
+  if ((T + bq - 1) / bq > 65535) HI_FAIL("%s: T=%d exceeds %d query rows", who, T, 65535 * bq);
+  const dim3 grid(Hq, (T + bq - 1) / bq);
   const hipStream_t s = (hipStream_t)stream;
-  const auto kern = D == 128 ? flash_prefill_kernel<128, kFpRG> : flash_prefill_kernel<64, kFpRG>;
-  const size_t lds = D == 128 ? FpSmem<128, kFpRG>::kBytes : FpSmem<64, kFpRG>::kBytes;
-  const int bpc = hi_blocks_per_cu(reinterpret_cast<const void*>(kern), 128 * kFpRG, lds);  // lifts the LDS limit
+  const auto kern = D == 128 ? (small ? flash_prefill_kernel<128, 2> : flash_prefill_kernel<128, kFpRG>)
+                             : (small ? flash_prefill_kernel<64, 2> : flash_prefill_kernel<64, kFpRG>);
+  const size_t lds = D == 128 ? (small ? FpSmem<128, 2>::kBytes : FpSmem<128, kFpRG>::kBytes)
+                              : (small ? FpSmem<64, 2>::kBytes : FpSmem<64, kFpRG>::kBytes);
+  const int bpc = hi_blocks_per_cu(reinterpret_cast<const void*>(kern), 64 * 2 * rg, lds);  // lifts the LDS limit
   if (bpc < 0) return -2;
   if (bpc == 0) HI_FAIL("%s: the kernel does not fit on a CU", who);
-  hipLaunchKernelGGL(kern, grid, dim3(128 * kFpRG), lds, s, (const f16*)q, (int64_t)ldq, (const f16*)kc, (const f16*)vc,
-                     max_seq, (f16*)out, (int64_t)ldo, T, p0, Hq, Hkv, scale_log2, lse);
+  hipLaunchKernelGGL(kern, grid, dim3(64 * 2 * rg), lds, s, (const f16*)q, (int64_t)ldq, (const f16*)kc,
+                     (const f16*)vc, max_seq, (f16*)out, (int64_t)ldo, T, p0, Hq, Hkv, scale_log2, lse);
   HI_TRY(hipGetLastError());
   return 0;
 }

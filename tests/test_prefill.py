@@ -130,6 +130,24 @@ def test_flash_prefill_tile_edges(hi, O, D, p0):
         check(f"flash prefill lse D={D} T={T} p0={p0}", host(lse), ref_lse, 1e-4, 1e-5)
 
 
+@pytest.mark.parametrize("D,Hq,T,p0", [(128, 32, 512, 0), (128, 32, 513, 0), (64, 32, 1024, 0), (64, 32, 1025, 0),
+                                        (64, 32, 512, 600), (64, 32, 513, 600)])
+def test_flash_prefill_row_block_rule(hi, O, D, Hq, T, p0):
+    """Both sides of the rule that gives small grids 64-row blocks (256 CUs: up to 256 of them at
+    D = 128, 512 at D = 64 when the prompt is longer than its prefix). Sampled rows against the
+    oracle, whose row t depends only on q[t] and the cache."""
+    r = rng(1290 + D + T + p0)
+    Hkv, S = 8, p0 + T
+    kc = r.standard_normal((Hkv, S, D)).astype(np.float16)
+    vc = r.standard_normal((Hkv, S, D)).astype(np.float16)
+    q = r.standard_normal((T, Hq * D)).astype(np.float16)
+    out, lse = hi.flash_prefill_lse(cuda(q), cuda(kc), cuda(vc), T, p0, Hq, Hkv)
+    for t in sorted({0, 1, 63, 64, 127, 128, T // 2, T - 2, T - 1}):
+        ref, ref_lse = O.flash_prefill(q[t:t + 1], kc, vc, 1, p0 + t, Hq, Hkv, lse=True)
+        check(f"flash prefill row {t} D={D} T={T} p0={p0}", host(out)[t:t + 1], ref, 2e-3, 1e-2)
+        check(f"flash prefill lse row {t}", host(lse)[:, t:t + 1], ref_lse, 1e-4, 1e-5)
+
+
 def test_flash_prefill_fused_qkv_rows_and_lse(hi, O):
     """q read in place from the rows of a fused qkv buffer (ldq = (Hq + 2 Hkv) D), output into a
     padded buffer (ldo > Hq D, the padding untouched), lse against the oracle's."""
