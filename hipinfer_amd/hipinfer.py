@@ -126,9 +126,22 @@ def ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def _addr(t):
+    """ptr() as the plain integer ctypes converts by itself (the wrappers' own calls)."""
+    return None if t is None else t.data_ptr()
+
+
+def _stream():
+    """torch's current HIP stream as an integer. torch.cuda.current_stream() builds a Stream object
+    and takes 3 us, a third of a small call; the raw handle takes 0.1."""
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def cur_stream():
     """torch's current HIP stream, as the library's `stream` argument."""
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_stream())
 
 
 def check_rc(rc, what):
@@ -180,7 +193,7 @@ def rmsnorm(x, w, eps=1e-5, out=None):
         _need("rmsnorm", t, torch.float16)
     if not (x.is_contiguous() and y.is_contiguous()):
         raise ValueError("hipinfer_amd.rmsnorm: rows of x and out must be packed")
-    check_rc(lib.hi_rmsnorm(ptr(x), ptr(w), ptr(y), x.shape[0], x.shape[1], eps, cur_stream()), "rmsnorm")
+    check_rc(lib.hi_rmsnorm(_addr(x), _addr(w), _addr(y), x.shape[0], x.shape[1], eps, _stream()), "rmsnorm")
     return y
 
 
@@ -196,9 +209,9 @@ def gemv(x, W, out=None, normw=None, eps=1e-5, epi=0, scales=None):
     if out is None:
         out = _alloc_rows(x, M, N // 2 if epi == 2 else N)
     _need("gemv", out, torch.float16, 2, rows=True)
-    head = (ptr(x), x.stride(0), ptr(normw), eps, ptr(W))
-    tail = (ptr(out), out.stride(0), M, N, K, epi, cur_stream())
-    rc = lib.hi_gemv_w8(*head, ptr(scales), *tail) if q8 else lib.hi_gemv(*head, *tail)
+    head = (_addr(x), x.stride(0), _addr(normw), eps, _addr(W))
+    tail = (_addr(out), out.stride(0), M, N, K, epi, _stream())
+    rc = lib.hi_gemv_w8(*head, _addr(scales), *tail) if q8 else lib.hi_gemv(*head, *tail)
     check_rc(rc, "gemv")
     return out
 
@@ -216,10 +229,10 @@ def gemv_qkv_rope(x, W, normw, Hq, Hkv, cs, pos, kc, vc, out, bias=None, eps=1e-
     _need("gemv_qkv_rope", bias, torch.float16, 1, optional=True)
     M, K = x.shape
     D, max_seq = kc.shape[3], kc.shape[2]
-    head = (ptr(x), x.stride(0), ptr(normw), eps, ptr(W))
-    tail = (ptr(bias), ptr(out), out.stride(0), M, K, Hq, Hkv, D, ptr(cs), ptr(pos), ptr(kc), ptr(vc), max_seq,
-            cur_stream())
-    rc = lib.hi_gemv_qkv_rope_w8(*head, ptr(scales), *tail) if q8 else lib.hi_gemv_qkv_rope(*head, *tail)
+    head = (_addr(x), x.stride(0), _addr(normw), eps, _addr(W))
+    tail = (_addr(bias), _addr(out), out.stride(0), M, K, Hq, Hkv, D, _addr(cs), _addr(pos), _addr(kc), _addr(vc), max_seq,
+            _stream())
+    rc = lib.hi_gemv_qkv_rope_w8(*head, _addr(scales), *tail) if q8 else lib.hi_gemv_qkv_rope(*head, *tail)
     check_rc(rc, "gemv_qkv_rope")
     return out
 
@@ -235,9 +248,9 @@ def gemm(A, W, out=None, epi=0, bias=None, scales=None):
     if out is None:
         out = _alloc_rows(A, M, N // 2 if epi == 2 else N)
     _need("gemm", out, torch.float16, 2, rows=True)
-    head = (ptr(A), A.stride(0), ptr(W))
-    tail = (ptr(bias), ptr(out), out.stride(0), M, N, K, epi, cur_stream())
-    rc = lib.hi_gemm_w8(*head, ptr(scales), *tail) if q8 else lib.hi_gemm(*head, *tail)
+    head = (_addr(A), A.stride(0), _addr(W))
+    tail = (_addr(bias), _addr(out), out.stride(0), M, N, K, epi, _stream())
+    rc = lib.hi_gemm_w8(*head, _addr(scales), *tail) if q8 else lib.hi_gemm(*head, *tail)
     check_rc(rc, "gemm")
     return out
 
@@ -255,8 +268,8 @@ def gemm_rmsnorm(A, W, x, normw, eps=1e-5, out=None, scales=None):
     if not (x.is_contiguous() and y.is_contiguous()):
         raise ValueError("hipinfer_amd.gemm_rmsnorm: rows of x and out must be packed")
     M, K = A.shape
-    check_rc(lib.hi_gemm_residual_rmsnorm(ptr(A), A.stride(0), ptr(W), ptr(scales), ptr(x), M, W.shape[0], K,
-                                          ptr(normw), eps, ptr(y), cur_stream()), "gemm_rmsnorm")
+    check_rc(lib.hi_gemm_residual_rmsnorm(_addr(A), A.stride(0), _addr(W), _addr(scales), _addr(x), M, W.shape[0], K,
+                                          _addr(normw), eps, _addr(y), _stream()), "gemm_rmsnorm")
     return y
 
 
@@ -270,8 +283,8 @@ def gemm_noalloc(A, W, out, epi=0, bias=None, scales=None):
     _need("gemm_noalloc", bias, torch.float16, 1, optional=True)
     _need("gemm_noalloc", out, torch.float16, 2, rows=True)
     M, K = A.shape
-    check_rc(lib.hi_gemm_noalloc(ptr(A), A.stride(0), ptr(W), ptr(scales), ptr(bias), ptr(out), out.stride(0), M,
-                                 W.shape[0], K, epi, cur_stream()), "gemm_noalloc")
+    check_rc(lib.hi_gemm_noalloc(_addr(A), A.stride(0), _addr(W), _addr(scales), _addr(bias), _addr(out), out.stride(0), M,
+                                 W.shape[0], K, epi, _stream()), "gemm_noalloc")
     return out
 
 
@@ -280,10 +293,11 @@ def _routing(xn, M, k):
             torch.empty(M, k, dtype=torch.float32, device=xn.device))
 
 
-def _moe_work(xn, M, k, E, H, I, zeroed=False):
-    """The expert work buffer; moe_route_experts needs it zeroed (its first 2304 bytes are arrival
-    counters that must start consistent)."""
-    make = torch.zeros if zeroed else torch.empty
+def _moe_work(xn, M, k, E, H, I, route=False):
+    """The expert work buffer. Its first 2304 bytes hold the arrival counters of moe_route_experts'
+    one-row launch, which must start at zero; more rows use no counters, so their buffer (17 MB at 700
+    rows of a 32-expert layer, 9 us to fill) is left as it is."""
+    make = torch.zeros if route and M == 1 else torch.empty
     return make(lib.hi_moe_work_bytes(M, k, E, H, I), dtype=torch.uint8, device=xn.device)
 
 
@@ -294,8 +308,8 @@ def moe_router(xn, Wr, k, flags):
     _need("moe_router", Wr, torch.float16, 2, rows=True)
     M, H = xn.shape
     idx, w = _routing(xn, M, k)
-    check_rc(lib.hi_moe_router(ptr(xn), xn.stride(0), ptr(Wr), M, Wr.shape[0], H, k, flags, ptr(idx), ptr(w),
-                               cur_stream()), "moe_router")
+    check_rc(lib.hi_moe_router(_addr(xn), xn.stride(0), _addr(Wr), M, Wr.shape[0], H, k, flags, _addr(idx), _addr(w),
+                               _stream()), "moe_router")
     return idx, w
 
 
@@ -309,8 +323,8 @@ def moe_experts(xn, wgu, wdown, idx, w, x, flags, scale=1.0, path=0):
     M, H = xn.shape
     E, I, k = wgu.shape[0], wdown.shape[2], idx.shape[1]
     work = _moe_work(xn, M, k, E, H, I)
-    check_rc(lib.hi_moe_experts(ptr(xn), xn.stride(0), ptr(wgu), ptr(wdown), ptr(idx), ptr(w), M, E, k, H, I, flags,
-                                scale, ptr(x), x.stride(0), path, ptr(work), cur_stream()), "moe_experts")
+    check_rc(lib.hi_moe_experts(_addr(xn), xn.stride(0), _addr(wgu), _addr(wdown), _addr(idx), _addr(w), M, E, k, H, I, flags,
+                                scale, _addr(x), x.stride(0), path, _addr(work), _stream()), "moe_experts")
     return x
 
 
@@ -324,9 +338,9 @@ def moe_route_experts(xn, Wr, wgu, wdown, k, x, flags, scale=1.0):
     M, H = xn.shape
     E, I = wgu.shape[0], wdown.shape[2]
     idx, w = _routing(xn, M, k)
-    work = _moe_work(xn, M, k, E, H, I, zeroed=True)
-    check_rc(lib.hi_moe_route_experts(ptr(xn), xn.stride(0), ptr(Wr), ptr(wgu), ptr(wdown), M, E, k, H, I, flags,
-                                      scale, ptr(x), x.stride(0), ptr(idx), ptr(w), ptr(work), cur_stream()),
+    work = _moe_work(xn, M, k, E, H, I, route=True)
+    check_rc(lib.hi_moe_route_experts(_addr(xn), xn.stride(0), _addr(Wr), _addr(wgu), _addr(wdown), M, E, k, H, I, flags,
+                                      scale, _addr(x), x.stride(0), _addr(idx), _addr(w), _addr(work), _stream()),
              "moe_route_experts")
     return idx, w
 
@@ -344,8 +358,8 @@ def decode_attn(q, kc, vc, pos, Hq, Hkv, out=None, work=None):
         out = _alloc_rows(q, B, Hq * D)
     if work is None:
         work = torch.zeros(lib.hi_decode_work_bytes(B, Hq, Hkv, D), dtype=torch.uint8, device=q.device)
-    check_rc(lib.hi_decode_attn(ptr(q), q.stride(0), ptr(kc), ptr(vc), max_seq, ptr(pos), ptr(out), out.stride(0), B,
-                                Hq, Hkv, D, ptr(work), cur_stream()), "decode_attn")
+    check_rc(lib.hi_decode_attn(_addr(q), q.stride(0), _addr(kc), _addr(vc), max_seq, _addr(pos), _addr(out), out.stride(0), B,
+                                Hq, Hkv, D, _addr(work), _stream()), "decode_attn")
     return out
 
 
@@ -356,8 +370,8 @@ def rope_cache(qkv, Hq, Hkv, cs, kc, vc, pos=None, pos_base=0, slot_base=0):
     _need("rope_cache", qkv, torch.float16, 2, rows=True)
     _need("rope_cache", pos, torch.int32, 1, optional=True)
     D, max_seq = kc.shape[3], kc.shape[2]
-    check_rc(lib.hi_rope_cache(ptr(qkv), qkv.stride(0), qkv.shape[0], Hq, Hkv, D, ptr(cs), ptr(pos), pos_base,
-                               slot_base, ptr(kc), ptr(vc), max_seq, cur_stream()), "rope_cache")
+    check_rc(lib.hi_rope_cache(_addr(qkv), qkv.stride(0), qkv.shape[0], Hq, Hkv, D, _addr(cs), _addr(pos), pos_base,
+                               slot_base, _addr(kc), _addr(vc), max_seq, _stream()), "rope_cache")
 
 
 def _flash(q, kc, vc, T, p0, Hq, Hkv, out, lse):
@@ -367,11 +381,11 @@ def _flash(q, kc, vc, T, p0, Hq, Hkv, out, lse):
     D, max_seq = kc.shape[2], kc.shape[1]
     if out is None:
         out = _alloc_rows(q, T, Hq * D)
-    args = (ptr(q), q.stride(0), ptr(kc), ptr(vc), max_seq, ptr(out), out.stride(0), T, p0, Hq, Hkv, D)
+    args = (_addr(q), q.stride(0), _addr(kc), _addr(vc), max_seq, _addr(out), out.stride(0), T, p0, Hq, Hkv, D)
     if lse is None:
-        check_rc(lib.hi_flash_prefill(*args, cur_stream()), "flash_prefill")
+        check_rc(lib.hi_flash_prefill(*args, _stream()), "flash_prefill")
     else:
-        check_rc(lib.hi_flash_prefill_lse(*args, ptr(lse), cur_stream()), "flash_prefill_lse")
+        check_rc(lib.hi_flash_prefill_lse(*args, _addr(lse), _stream()), "flash_prefill_lse")
     return out
 
 
@@ -398,7 +412,7 @@ def argmax(logits, out=None):
     B, V = logits.shape
     if out is None:
         out = torch.empty(B, dtype=torch.int32, device=logits.device)
-    check_rc(lib.hi_argmax(ptr(logits), B, V, ptr(out), cur_stream()), "argmax")
+    check_rc(lib.hi_argmax(_addr(logits), B, V, _addr(out), _stream()), "argmax")
     return out
 
 
@@ -409,7 +423,7 @@ def embed(tok, table, out=None):
     V, H = table.shape
     if out is None:
         out = _alloc_rows(table, tok.shape[0], H)
-    check_rc(lib.hi_embed(ptr(tok), ptr(table), V, H, ptr(out), out.stride(0), tok.shape[0], cur_stream()), "embed")
+    check_rc(lib.hi_embed(_addr(tok), _addr(table), V, H, _addr(out), out.stride(0), tok.shape[0], _stream()), "embed")
     return out
 
 
@@ -423,7 +437,7 @@ def quantize_rows(w):
     N, K = w.shape
     q = torch.empty(N, K, dtype=torch.int8, device=w.device)
     s = torch.empty(N, dtype=torch.float16, device=w.device)
-    check_rc(lib.hi_quantize_rows(ptr(w), N, K, ptr(q), ptr(s), cur_stream()), "quantize_rows")
+    check_rc(lib.hi_quantize_rows(_addr(w), N, K, _addr(q), _addr(s), _stream()), "quantize_rows")
     return q, s
 
 
@@ -433,7 +447,7 @@ def dequantize_rows(q, s):
     _need("dequantize_rows", s, torch.float16, 1)
     q = q.contiguous()
     out = torch.empty(q.shape, dtype=torch.float16, device=q.device)
-    check_rc(lib.hi_dequantize_rows(ptr(q), ptr(s), q.shape[0], q.shape[1], ptr(out), cur_stream()), "dequantize_rows")
+    check_rc(lib.hi_dequantize_rows(_addr(q), _addr(s), q.shape[0], q.shape[1], _addr(out), _stream()), "dequantize_rows")
     return out
 
 
