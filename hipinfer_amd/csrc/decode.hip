@@ -4,19 +4,29 @@
 // reference's internal embed_kernel, kernels.cuh:1876-1881, called from decode_step api.cu:1900)
 // is exported as well so that a caller can assemble a whole decode step from C-ABI calls.
 //
-// Decode attention, one new token per sequence, for gfx950:
-//  * block = (split, kv head, sequence), 4 waves; every block serves all G query heads of its kv
-//    head, so the cache is read once per GQA group. A split covers a contiguous run of keys; the
-//    number of splits in use is derived on the device from pos[b], so a captured graph stays valid
-//    while the context grows;
-//  * a wave takes 64-key tiles: the tile's K rows go straight into LDS (1 KB per DMA instruction)
-//    and its V rows into registers, all in flight at once (the wave's first tile before anything
-//    else), so a tile costs one memory round trip; lane l then owns key t0 + l, reads its K row
-//    from LDS and computes the key's logit for every query head in fp32 with the query chunks in
-//    scalar registers (scalar loads, the same for every lane; q pre-scaled by log2(e) / sqrt(D),
-//    the reference's log2-domain softmax, kernels.cuh:1522);
-//  * online softmax per wave (max and sum over the 64 lanes), P.V with each lane owning D / 64
-//    output dims and the weights as fp16 key pairs through LDS, the 4 waves merged through LDS;
+// Decode attention, one new token per sequence, for gfx950. The cache is read once, so the floor is
+// its bytes; what lies above it is the chain of one launch (position, tiles, partials, counter,
+// merge) and, over ragged batches, the wait for the longest blocks:
+//  * block = (split, kv head, sequence); every block serves all G query heads of its kv head, so the
+//    cache is read once per GQA group. A split covers a contiguous run of keys; the number of splits
+//    in use is derived on the device from pos[b], so a captured graph stays valid while the context
+//    grows;
+//  * a wave takes 32-key tiles. Logits are S^T = K Q^T and the output O^T = V^T P^T, both on 16x16x32
+//    MFMAs with the group's heads as columns (1 to 8 of 16; the products are free beside the loads).
+//    K and V go straight from memory into operand registers: which key is which row of a K operand,
+//    and which dim which row of a V operand, is chosen so that the logits of a lane are its P operand
+//    and the V rows are read whole, the transpose being v_perms inside a lane. No LDS, no shuffle but
+//    the maximum's. A tile's registers are refilled for the next tile as soon as they are used (K
+//    behind the logits, V behind P.V), so a wave keeps 8 to 16 KB in flight;
+//  * logits are exact fp16 products in fp32 sums, scaled by log2(e) / sqrt(D) in fp32 (the
+//    reference's log2-domain softmax, kernels.cuh:1522); the weights are fp16 for P.V (as the
+//    reference's tensor-core path packs them, kernels.cuh:1455-1460) and fp32 in their sum;
+//  * online softmax per wave, the block's waves merged through LDS;
+//  * measured, cold caches, against one key per lane with v_dot2 and K through LDS (56-64 KB of it, so
+//    two blocks per CU and no overlap of loads with arithmetic inside a wave), us: 48 sequences of 100
+//    to 2000 keys, 32/8 heads of 128: 49.6 -> 43.5; 64 of 1000: 53 -> 49.8 (5.3 TB/s); 40 of 200 to
+//    1600, 32/4 heads of 64: 24.6 -> 15.4; one of 4001, 32/8 of 128: 11.7 -> 10.5; four of 700 to 800,
+//    32/4 of 64: 11.1 -> 7.4;
 //  * splits hand their partials (o, m, l) to the last-arriving block of their (sequence, kv head)
 //    with agent-coherent (sc1) stores and loads and a relaxed agent-scope counter, which the last
 //    block resets: no L2 writeback/invalidate fence (gfx950's agent-scope fence costs several
@@ -27,16 +37,11 @@
 #include "hi_common.h"
 #include "hi_internal.h"
 
-#ifndef HI_DA_WAVES
-#define HI_DA_WAVES 4
-#endif
-
 namespace {
 
 constexpr int kDecodeCounters = 4096;  // as api.cu:651: counters at a fixed offset, then partials
 constexpr int kDecodeMaxSplits = 64;
-constexpr int kDaTile = 64;  // keys per wave tile (one per lane)
-constexpr int kDaWaves = HI_DA_WAVES;  // waves per block
+constexpr int kDaTile = 32;  // keys per wave tile (one k step of P.V)
 
 __device__ __forceinline__ float ld_coherent(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -45,39 +50,49 @@ __device__ __forceinline__ void st_coherent(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// LDS of one block: the waves' K tiles and softmax weights while the keys stream, then (after a
-// barrier) the waves' partial results and the split merge's tables in the same bytes.
+// Maximum (or sum) over the four 16-lane rows of a wave, each lane with the lanes of its own column.
+template <bool MAX>
+__device__ __forceinline__ float rows_reduce(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = MAX ? fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])) : __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = MAX ? fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1])) : __uint_as_float(b[0]) + __uint_as_float(b[1]);
+#endif
+  return v;
+}
+
+// Splits in use for `len` keys when a launch has S per pair and S1 give every CU two blocks: of those,
+// one per 256 keys, but down to 128 keys a split while there are at most
+// 16 (what the merge requests in one round): shorter waves finish sooner, and more splits cost more
+// in the merge (one sequence of 4001 keys, 32/8 heads: 16 splits 10.8 us, 32 splits 12.5; of 2500: 16
+// 9.5, 10 9.9). Beyond them only for runs over 1024 keys, which would end a ragged batch late (30
+// sequences of 500 to 4000: 73 -> 71 us); at 512 keys a uniform batch of 64 x 1000 leaves a part-filled
+// last round (49.8 -> 54.7).
+__device__ __forceinline__ int splits_used(int len, int S, int S1) {
+  return max(min(S1, max((len + 255) / 256, min(16, (len + 127) / 128))), min(S, (len + 1023) / 1024));
+}
+
+// LDS of one block: the waves' partial results and the split merge's tables.
 template <int G, int D, int NWV>
 struct DaSmem {
-  static constexpr int CPR = D / 8;
-  struct Loop {
-    u32x4 ks[NWV][kDaTile * CPR];      // K tile, chunk c of row r at slot c ^ (r % CPR)
-    uint32_t ps[NWV][G][kDaTile / 2];  // softmax weights, fp16 pairs of keys
-  };
-  struct Merge {
-    float wo[NWV][G][D];
-    float sm[G][kDecodeMaxSplits], sw[G][kDecodeMaxSplits];
-  };
-  union {
-    Loop loop;
-    Merge merge;
-  };
+  float wo[NWV][G][D];
+  float wm[NWV][G], wl[NWV][G];
+  float sm[G][kDecodeMaxSplits], sw[G][kDecodeMaxSplits];
+  int is_last;
 };
 
 template <int G, int D, int NWV>
-__global__ void __launch_bounds__(NWV * 64) decode_attn_kernel(const f16* __restrict__ q, int ldq,
-                                                               const f16* __restrict__ kc, const f16* __restrict__ vc,
-                                                               int max_seq, int Hkv, const int* __restrict__ pos,
-                                                               float* part, int* counters, int S, f16* __restrict__ out,
-                                                               int ldo, float scale_log2, int kv_slot) {
-  constexpr int DPL = D / 64;        // output dims per lane
-  constexpr int CPR = D / 8;         // 16-byte chunks of a K row
-  constexpr int RPI = 64 / CPR;      // K rows per 1 KB DMA instruction
-  constexpr int BK = NWV * kDaTile;  // keys per block pass
+__global__ void __launch_bounds__(NWV * 64, 3) decode_attn_kernel(
+    const f16* __restrict__ q, int ldq, const f16* __restrict__ kc, const f16* __restrict__ vc, int max_seq, int Hkv,
+    const int* __restrict__ pos, float* part, int* counters, int S, int S1, f16* __restrict__ out,
+    int ldo, float scale_log2, int kv_slot) {
+  constexpr int KS = D / 32;               // k steps of a logits product
+  constexpr int DL = D / 16;               // V dims (and P.V products) per lane
+  constexpr int BK = NWV * kDaTile;        // keys per block pass
   constexpr int NT = NWV * 64;
+  typedef typename std::conditional<DL == 8, u32x4, u32x2>::type VT;
   __shared__ DaSmem<G, D, NWV> sh;
-  __shared__ float wm[NWV][G], wl[NWV][G];
-  __shared__ int is_last;
   // blocks in split-major order: the splits a sequence uses (split < S_eff) come first in dispatch
   // order, so they spread over the CUs instead of sharing them with blocks that exit at once
   const int nhb = gridDim.x / S;  // (sequence, kv head) pairs
@@ -85,7 +100,7 @@ __global__ void __launch_bounds__(NWV * 64) decode_attn_kernel(const f16* __rest
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int Hq = Hkv * G;
   const int len = min(pos[b] + 1, max_seq);
-  const int S_eff = min(S, (len + BK - 1) / BK);
+  const int S_eff = splits_used(len, S, S1);
   if (split >= S_eff) return;
   const int chunk = (len + S_eff - 1) / S_eff;
   const int start = split * chunk, end = min(len, start + chunk);
@@ -97,135 +112,120 @@ __global__ void __launch_bounds__(NWV * 64) decode_attn_kernel(const f16* __rest
   const __amdgpu_buffer_rsrc_t v_rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(Vh), (short)0, end * D * 2, 0x00020000);
 
-  // a tile's K rows, 1 KB per instruction straight into LDS, swizzled so that the one-key-per-lane
-  // reads below are conflict-free; rows at or past the split's end read as zeros through the
-  // buffer bounds.
-  auto issue_tile = [&](int t0) {
+  const int r = lane & 15, fk = lane >> 4;
+  // Logits as S^T = K Q^T (16x16x32): A row r of block a is the tile's key 8 (r / 4) + 4 a + r % 4,
+  // so lane group fk of the C layout ends up with keys 8 fk .. 8 fk + 7 of head r, in order: the B
+  // operand of the 32-key P.V product, without a shuffle. Rows at or past the split's end read as
+  // zeros through the buffer bounds.
+  const unsigned k_off = (8 * (r >> 2) + (r & 3)) * D * 2 + 16 * fk;
+  // V: lane (r, fk) loads dims DL r .. of keys 8 fk + i, whole rows per instruction; P.V product n
+  // takes dim n of every lane's DL as its A row, over the lane's 8 keys (D = 64: 8-byte loads of 4 dims).
+  const unsigned v_off = 8 * fk * D * 2 + DL * 2 * r;
+  u32x4 kf[2][KS];
+  VT vf[8];
+  auto load_k = [&](int t0) {
 #pragma unroll
-    for (int i = 0; i < kDaTile / RPI; i++) {
-      const int r = i * RPI + lane / CPR, c = (lane % CPR) ^ (r % CPR);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rs, (__attribute__((address_space(3))) void*)&sh.loop.ks[wave][i * 64],
-                                               16, ((t0 + r) * D + 8 * c) * 2, 0, 0, 0);
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+        kf[a][s] = __builtin_amdgcn_raw_buffer_load_b128(k_rs, k_off + (unsigned)t0 * (D * 2) + 4 * a * D * 2 + 64 * s,
+                                                         0, 0);
+  };
+  auto load_v = [&](int t0) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const unsigned off = v_off + (unsigned)t0 * (D * 2) + i * D * 2;
+      if constexpr (DL == 8) vf[i] = __builtin_amdgcn_raw_buffer_load_b128(v_rs, off, 0, 0);
+      else vf[i] = __builtin_amdgcn_raw_buffer_load_b64(v_rs, off, 0, 0);
     }
   };
   const int t_first = start + wave * kDaTile;
-  if (t_first < end) issue_tile(t_first);
-  // the group's query rows are read in the loop with scalar loads (the same for every lane): no
-  // LDS copy, no vector registers, no barrier before a wave's first tile
-  const f16* qg = q + (int64_t)b * ldq + hk * G * D;
-
-  float m[G], l[G], o[G][DPL];
+  const f16* qg = q + (int64_t)b * ldq + (hk * G + (r < G ? r : 0)) * D + 8 * fk;
+  float m = -__builtin_huge_valf(), l = 0.f;  // of head r; l over this lane's keys only
+  f32x4 o[DL];                                // O^T: dim DL (4 fk + i) + n of head r in o[n][i]
 #pragma unroll
-  for (int g = 0; g < G; g++) {
-    m[g] = -__builtin_huge_valf();
-    l[g] = 0.f;
+  for (int n = 0; n < DL; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (t_first < end) {
+    load_k(t_first);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 qf[KS];
 #pragma unroll
-    for (int d = 0; d < DPL; d++) o[g][d] = 0.f;
-  }
-
-  for (int t0 = t_first; t0 < end; t0 += BK) {
-    // keeps the query loads inside the loop: hoisted, they would need G * D / 2 scalar registers
-    asm volatile("" ::: "memory");
-    const int n = min(kDaTile, end - t0);
-    const bool valid = lane < n;
-    if (t0 != t_first) issue_tile(t0);
-    // the tile's V rows into registers (lane l: dims l*DPL..), in flight with its K rows
-    typedef typename std::conditional<DPL == 2, uint32_t, uint16_t>::type VT;
-    VT vv[kDaTile];
+    for (int s = 0; s < KS; s++) qf[s] = *reinterpret_cast<const u32x4*>(qg + 32 * s);
+    load_v(t_first);
+    // One tile; the next tile's K is requested as soon as this one's is used, and so is its V.
+    auto tile = [&](int t0, auto last) {
+      constexpr bool LAST = decltype(last)::value;
+      f32x4 sc[2];
 #pragma unroll
-    for (int jj = 0; jj < kDaTile; jj++) {
-      const int off = ((t0 + jj) * D + lane * DPL) * 2;
-      if constexpr (DPL == 2) vv[jj] = __builtin_amdgcn_raw_buffer_load_b32(v_rs, off, 0, 0);
-      else vv[jj] = __builtin_amdgcn_raw_buffer_load_b16(v_rs, off, 0, 0);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): K in LDS, V in registers
-    __builtin_amdgcn_wave_barrier();
-    u32x4 kv[CPR];
+      for (int a = 0; a < 2; a++) {
+        sc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < CPR; c++) kv[c] = sh.loop.ks[wave][lane * CPR + (c ^ (lane % CPR))];
-
-    // logits: fp16 q . fp16 k with exact products and fp32 sums (v_dot2_f32_f16), then the
-    // log2(e) / sqrt(D) scale once per logit (the reference's log2-domain softmax, kernels.cuh:1522)
-    float s[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) s[g] = 0.f;
-#pragma unroll
-    for (int c = 0; c < CPR; c++) {
-#pragma unroll
-      for (int g = 0; g < G; g++) {
-        const u32x4 qv = *reinterpret_cast<const u32x4*>(qg + g * D + 8 * c);
-#pragma unroll
-        for (int p = 0; p < 4; p++) s[g] = dot2(as_h2(qv[p]), as_h2(kv[c][p]), s[g]);
+        for (int s = 0; s < KS; s++)
+          sc[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kf[a][s]),
+                                                         __builtin_bit_cast(f16x8, qf[s]), sc[a], 0, 0, 0);
       }
-    }
-#pragma unroll
-    for (int g = 0; g < G; g++) s[g] *= scale_log2;
-    float p_[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      const float sv = valid ? s[g] : -__builtin_huge_valf();
-      const float mn = fmaxf(m[g], wave_max(sv));  // finite: every tile has a valid key
-      p_[g] = valid ? exp2f(sv - mn) : 0.f;
-      const float a = exp2f(m[g] - mn);  // 0 on the first tile (m = -inf)
-      l[g] = l[g] * a + wave_sum(p_[g]);
-      m[g] = mn;
-#pragma unroll
-      for (int d = 0; d < DPL; d++) o[g][d] *= a;
-    }
-    // P.V: lane l owns dims l*DPL..; the weights go through LDS as fp16 pairs of consecutive keys
-    // (the precision of the reference's tensor-core path, which packs P to half for its MMA,
-    // kernels.cuh:1455-1460), and each pair of keys meets its two V values per dim in one
-    // v_dot2_f32_f16. A wave's LDS accesses complete in order, so its writes are visible to its
-    // later reads.
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      const float hi = __shfl_xor(p_[g], 1, 64);  // the neighbouring key's weight
-      if ((lane & 1) == 0) sh.loop.ps[wave][g][lane >> 1] = as_u32(f16x2{(f16)p_[g], (f16)hi});
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int j8 = 0; j8 < kDaTile; j8 += 8) {
-      if (j8 < n) {  // uniform over the wave; keys past n have p = 0 and V = 0
-        u32x4 pw[G];
-#pragma unroll
-        for (int g = 0; g < G; g++) pw[g] = *reinterpret_cast<const u32x4*>(&sh.loop.ps[wave][g][j8 / 2]);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const int j = j8 + 2 * k;
-          if constexpr (DPL == 2) {
-            // (v_j[d0], v_j[d1]), (v_j+1[d0], v_j+1[d1]) -> (v_j[d0], v_j+1[d0]), (v_j[d1], v_j+1[d1])
-            const uint32_t a0 = vv[j], a1 = vv[j + 1];
-            const f16x2 v0 = as_h2(__builtin_amdgcn_perm(a1, a0, 0x05040100u));
-            const f16x2 v1 = as_h2(__builtin_amdgcn_perm(a1, a0, 0x07060302u));
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-              o[g][0] = dot2(as_h2(pw[g][k]), v0, o[g][0]);
-              o[g][1] = dot2(as_h2(pw[g][k]), v1, o[g][1]);
-            }
-          } else {
-            const f16x2 v0 = as_h2((uint32_t)vv[j] | ((uint32_t)vv[j + 1] << 16));
-#pragma unroll
-            for (int g = 0; g < G; g++) o[g][0] = dot2(as_h2(pw[g][k]), v0, o[g][0]);
-          }
-        }
+      if constexpr (!LAST) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(t0 + BK);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+      float p[8];
+      float mx = -__builtin_huge_valf();
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        p[k] = sc[k >> 2][k & 3] * scale_log2;
+        if (LAST && t0 + 8 * fk + k >= end) p[k] = -__builtin_huge_valf();
+        mx = fmaxf(mx, p[k]);
+      }
+      const float mn = fmaxf(m, rows_reduce<true>(mx));  // finite: every tile has a valid key
+      const float alpha = exp2f(m - mn);                 // 0 on the first tile (m = -inf)
+      m = mn;
+      float ps = 0.f;
+      f16x8 pf;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        p[k] = exp2f(p[k] - mn);
+        ps += p[k];
+        pf[k] = (f16)p[k];
+      }
+      l = __builtin_fmaf(l, alpha, ps);
+#pragma unroll
+      for (int n = 0; n < DL; n++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[n][i] *= alpha;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < DL; n++) {
+        u32x4 w;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          w[k] = __builtin_amdgcn_perm(vf[2 * k + 1][n >> 1], vf[2 * k][n >> 1], n & 1 ? 0x07060302u : 0x05040100u);
+        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), pf, o[n], 0, 0, 0);
+      }
+      if constexpr (!LAST) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(t0 + BK);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    int t0 = t_first;
+    for (; t0 + BK < end; t0 += BK) tile(t0, std::false_type{});
+    tile(t0, std::true_type{});
   }
+  l = rows_reduce<false>(l);
 
   // ---- merge the block's waves (a wave without keys has m = -inf and weight 0)
-  __syncthreads();  // every wave is done with the loop's LDS before it is reused
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-    if (lane == 0) {
-      wm[wave][g] = m[g];
-      wl[wave][g] = l[g];
+  if (r < G) {
+    if (fk == 0) {
+      sh.wm[wave][r] = m;
+      sh.wl[wave][r] = l;
     }
 #pragma unroll
-    for (int d = 0; d < DPL; d++) sh.merge.wo[wave][g][lane * DPL + d] = o[g][d];
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int n = 0; n < DL; n += 4)
+        *reinterpret_cast<f32x4*>(&sh.wo[wave][r][DL * (4 * fk + i) + n]) =
+            f32x4{o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]};
   }
   __syncthreads();
   const bool single = S_eff == 1;
@@ -234,13 +234,13 @@ __global__ void __launch_bounds__(NWV * 64) decode_attn_kernel(const f16* __rest
     const int g = i / D, d = i % D;
     float M = -__builtin_huge_valf();
 #pragma unroll
-    for (int w = 0; w < NWV; w++) M = fmaxf(M, wm[w][g]);
+    for (int w = 0; w < NWV; w++) M = fmaxf(M, sh.wm[w][g]);
     float L = 0.f, O = 0.f;
 #pragma unroll
     for (int w = 0; w < NWV; w++) {
-      const float f = wm[w][g] == -__builtin_huge_valf() ? 0.f : exp2f(wm[w][g] - M);
-      L = __builtin_fmaf(wl[w][g], f, L);
-      O = __builtin_fmaf(sh.merge.wo[w][g][d], f, O);
+      const float f = sh.wm[w][g] == -__builtin_huge_valf() ? 0.f : exp2f(sh.wm[w][g] - M);
+      L = __builtin_fmaf(sh.wl[w][g], f, L);
+      O = __builtin_fmaf(sh.wo[w][g][d], f, O);
     }
     if (single) {
       out[(int64_t)b * ldo + (hk * G + g) * D + d] = (f16)(O / L);
@@ -259,11 +259,11 @@ __global__ void __launch_bounds__(NWV * 64) decode_attn_kernel(const f16* __rest
   if (tid == 0) {
     int* ctr = counters + b * Hkv + hk;
     const int done = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    is_last = done == S_eff - 1;
-    if (is_last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+    sh.is_last = done == S_eff - 1;
+    if (sh.is_last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
   }
   __syncthreads();
-  if (!is_last) return;
+  if (!sh.is_last) return;
   // ---- the last block merges the S_eff splits of every head of its group, in split order. The
   //      (m, l) pairs and the first 16 splits' partial outputs are requested in one round; the
   //      split weights exp2(m_s - M) / L are formed once per head while those loads are in flight.
@@ -280,19 +280,19 @@ __global__ void __launch_bounds__(NWV * 64) decode_attn_kernel(const f16* __rest
   for (int i = tid; i < G * S_eff; i += NT) {
     const int g = i / S_eff, s2 = i - g * S_eff;
     const float* pp = po + (((int64_t)b * Hq + hk * G + g) * kDecodeMaxSplits + s2) * (D + 2);
-    sh.merge.sm[g][s2] = ld_coherent(pp + D);
-    sh.merge.sw[g][s2] = ld_coherent(pp + D + 1);
+    sh.sm[g][s2] = ld_coherent(pp + D);
+    sh.sw[g][s2] = ld_coherent(pp + D + 1);
   }
   __syncthreads();
   for (int g = wave; g < G; g += NWV) {
     float M = -__builtin_huge_valf();
-    for (int s2 = lane; s2 < S_eff; s2 += 64) M = fmaxf(M, sh.merge.sm[g][s2]);
+    for (int s2 = lane; s2 < S_eff; s2 += 64) M = fmaxf(M, sh.sm[g][s2]);
     M = wave_max(M);
     float Lp = 0.f;
     for (int s2 = lane; s2 < S_eff; s2 += 64)
-      Lp = __builtin_fmaf(sh.merge.sw[g][s2], exp2f(sh.merge.sm[g][s2] - M), Lp);
+      Lp = __builtin_fmaf(sh.sw[g][s2], exp2f(sh.sm[g][s2] - M), Lp);
     const float Lt = wave_sum(Lp);
-    for (int s2 = lane; s2 < S_eff; s2 += 64) sh.merge.sw[g][s2] = exp2f(sh.merge.sm[g][s2] - M) / Lt;
+    for (int s2 = lane; s2 < S_eff; s2 += 64) sh.sw[g][s2] = exp2f(sh.sm[g][s2] - M) / Lt;
   }
   __syncthreads();
 #pragma unroll
@@ -303,34 +303,40 @@ __global__ void __launch_bounds__(NWV * 64) decode_attn_kernel(const f16* __rest
       const float* pp = po + ((int64_t)b * Hq + hk * G + g) * kDecodeMaxSplits * (D + 2) + d;
       float O = 0.f;
 #pragma unroll
-      for (int k = 0; k < 16; k++) O = __builtin_fmaf(v0[e][k], k < S_eff ? sh.merge.sw[g][k] : 0.f, O);
+      for (int k = 0; k < 16; k++) O = __builtin_fmaf(v0[e][k], k < S_eff ? sh.sw[g][k] : 0.f, O);
       for (int s0 = 16; s0 < S_eff; s0 += 16) {
         float v[16];
 #pragma unroll
         for (int k = 0; k < 16; k++) v[k] = ld_coherent(pp + (int64_t)min(s0 + k, S_eff - 1) * (D + 2));
 #pragma unroll
-        for (int k = 0; k < 16; k++) O = __builtin_fmaf(v[k], s0 + k < S_eff ? sh.merge.sw[g][s0 + k] : 0.f, O);
+        for (int k = 0; k < 16; k++) O = __builtin_fmaf(v[k], s0 + k < S_eff ? sh.sw[g][s0 + k] : 0.f, O);
       }
       out[(int64_t)b * ldo + (hk * G + g) * D + d] = (f16)O;
     }
   }
 }
 
-// Splits per (sequence, kv head): enough blocks for two per CU (as api.cu:643-646), at most 64;
-// the kernel uses min(S, ceil(len / 256)) of them.
-int decode_splits(int B, int Hkv, int cus) {
-  const int S = (2 * cus + B * Hkv - 1) / (B * Hkv);
-  return S < 1 ? 1 : S > kDecodeMaxSplits ? kDecodeMaxSplits : S;
-}
+// Splits of a (sequence, kv head) pair that give every CU two blocks (as api.cu:643-646), at most the
+// work buffer's 64.
+int decode_splits(int B, int Hkv, int cus) { return min((2 * cus + B * Hkv - 1) / (B * Hkv), kDecodeMaxSplits); }
 
 template <int D>
 int decode_attn_d(int G, dim3 grid, hipStream_t s, const f16* q, int ldq, const f16* kc, const f16* vc, int max_seq,
-                  int Hkv, const int* pos, float* part, int* counters, int S, f16* out, int ldo, float sl2,
+                  int Hkv, const int* pos, float* part, int* counters, int S, int S1, f16* out, int ldo, float sl2,
                   int kv_slot) {
-#define HI_DA(g)                                                                                                      \
-  case g:                                                                                                             \
-    hipLaunchKernelGGL((decode_attn_kernel<g, D, kDaWaves>), grid, dim3(kDaWaves * 64), 0, s, q, ldq, kc, vc, max_seq, \
-                       Hkv, pos, part, counters, S, out, ldo, sl2, kv_slot);                                          \
+  // 8 waves where S1 is 16 or more (at most about an eighth as many pairs as CUs): a launch this
+  // small is a chain of latencies, and a block of 256 keys is then one tile per wave (one sequence of
+  // 2500 keys 9.45 -> 9.0 us, of 8000 14.8 -> 13.8, four of 700 to 800 at D = 64 8.1 -> 7.4); with more
+  // pairs 4 waves balance better (40 sequences of 300 to 2400, 12/2 heads: 19.5 against 25.5).
+  const bool wide = S1 >= 16;
+#define HI_DA(g)                                                                                              \
+  case g:                                                                                                     \
+    if (wide)                                                                                                 \
+      hipLaunchKernelGGL((decode_attn_kernel<g, D, 8>), grid, dim3(512), 0, s, q, ldq, kc, vc, max_seq, Hkv,  \
+                         pos, part, counters, S, S1, out, ldo, sl2, kv_slot);                                     \
+    else                                                                                                      \
+      hipLaunchKernelGGL((decode_attn_kernel<g, D, 4>), grid, dim3(256), 0, s, q, ldq, kc, vc, max_seq, Hkv,  \
+                         pos, part, counters, S, S1, out, ldo, sl2, kv_slot);                                     \
     break;
   switch (G) {
     HI_DA(1) HI_DA(2) HI_DA(3) HI_DA(4) HI_DA(5) HI_DA(6) HI_DA(7) HI_DA(8)
@@ -468,7 +474,7 @@ static int decode_attn_run(const void* q, int ldq, const void* kc, const void* v
     HI_FAIL("%s: q, kc and vc must be 16-byte aligned and ldq a multiple of 8", who);
   if (ldq < Hq * D || ldo < Hq * D) HI_FAIL("%s: ldq %d / ldo %d < Hq * D = %d", who, ldq, ldo, Hq * D);
   // one sequence (kv_slot >= 0): a batch of one's split count, so every row matches that decode
-  const int S = decode_splits(kv_slot >= 0 ? 1 : B, Hkv, d->cus);
+  const int S1 = decode_splits(kv_slot >= 0 ? 1 : B, Hkv, d->cus), S = min(2 * S1, kDecodeMaxSplits);
   const float sl2 = 1.4426950408889634f / sqrtf((float)D);
   const dim3 grid(S * Hkv * B);  // split-major: (split, sequence, kv head)
   int* counters = (int*)work;
@@ -476,9 +482,9 @@ static int decode_attn_run(const void* q, int ldq, const void* kc, const void* v
   const hipStream_t st = (hipStream_t)s;
   if (D == 64)
     return decode_attn_d<64>(Hq / Hkv, grid, st, (const f16*)q, ldq, (const f16*)kc, (const f16*)vc, max_seq, Hkv, pos,
-                             part, counters, S, (f16*)out, ldo, sl2, kv_slot);
+                             part, counters, S, S1, (f16*)out, ldo, sl2, kv_slot);
   return decode_attn_d<128>(Hq / Hkv, grid, st, (const f16*)q, ldq, (const f16*)kc, (const f16*)vc, max_seq, Hkv, pos,
-                            part, counters, S, (f16*)out, ldo, sl2, kv_slot);
+                            part, counters, S, S1, (f16*)out, ldo, sl2, kv_slot);
 }
 
 // out[b, h*D : (h+1)*D] = softmax(q_h . K[0..pos[b]] / sqrt(D)) V for every query head h of

@@ -65,6 +65,30 @@ def test_decode_attn_batch64(hi, O):
     check("decode attn B=64 lens=1024..205", got, ref, 2e-3, 1e-2)
 
 
+@pytest.mark.parametrize("D,Hkv,G", [(64, 8, 8), (128, 8, 4), (128, 2, 5)], ids=["D64-G8", "D128-G4", "D128-G5"])
+@pytest.mark.parametrize("B", [1, 3, 24, 70], ids=lambda b: f"B{b}")
+def test_decode_attn_tile_and_split_edges(hi, O, D, Hkv, G, B):
+    """Lengths at the edges of a wave's 32 keys, a block pass of 4 or 8 waves (128 and 256 keys) and
+    the split rule's steps (128, 256 and 1024 keys, 16 splits), at batches of both block widths, with
+    infinities and NaN in the cache behind every length: keys past it must not take part."""
+    edges = [1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 1023, 1024, 1025, 2047, 2048, 2049, 2079, 2080]
+    S, Hq = 2080, Hkv * G
+    for first in range(len(edges) if B == 1 else 1):
+        lens = [edges[(first + 5 * b) % len(edges)] for b in range(B)]
+        r = rng(640 + B + first)
+        q = r.standard_normal((B, Hq * D)).astype(np.float16)
+        kc = np.empty((B, Hkv, S, D), np.float16)
+        vc = np.empty((B, Hkv, S, D), np.float16)
+        kc[:] = r.standard_normal((1, Hkv, S, D))
+        vc[:] = r.standard_normal((1, Hkv, S, D))
+        for b, n in enumerate(lens):
+            kc[b, :, n:] = np.inf
+            vc[b, :, n:] = np.nan
+        pos = np.array(lens, np.int32) - 1
+        got = host(hi.decode_attn(cuda(q), cuda(kc), cuda(vc), cuda(pos), Hq, Hkv))
+        check(f"decode attn D={D} G={G} B={B} lens={lens[:4]}", got, O.decode_attn(q, kc, vc, pos, Hq, Hkv), 2e-3, 1e-2)
+
+
 def test_decode_work_reuse(hi, O):
     """One zeroed work buffer for launches of decreasing and increasing batch: the split counters
     must be left zeroed and never land in a larger launch's partials. One kv head per sequence
