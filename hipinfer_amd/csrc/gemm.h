@@ -793,6 +793,8 @@ constexpr bool gemm_cfg_fits(int c, bool q8, int K) {
 // 64 rows each), so each expert's weights are streamed once; a 64-row tile split most experts into
 // two row tiles, each streaming the same weights.
 constexpr int kGrpBM = 128, kGrpBN = 128, kGrpWM = 2, kGrpWN = 2, kGrpStages = 4, kGrpBK = 64;
+// Tall variant for experts of more than 128 rows (8 waves, three stages of 48 KB).
+constexpr int kGrpTallBM = 256, kGrpTallWM = 4, kGrpTallStages = 3;
 // Ring stages of a config's A and W tiles. The 64-deep 256 x 256 and 256 x 192 tiles hold one more
 // stage for W than for A (in fp16, 256 x 256 fills the CU's 160 KB with it): with two stages of
 // both, each tile's DMA has less than one tile of MFMA work to land and must go out in one burst;

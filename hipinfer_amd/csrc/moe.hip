@@ -350,13 +350,14 @@ __global__ void __launch_bounds__(kMoeWaves * 64) moe_gemv_down_kernel(const f16
 
 // ------------------------------------------------------------------ grouped path
 // Counting sort of the n (token, slot) pairs by expert, by one block of kSortThreads: off[E+1] the
-// exclusive prefix of the per-expert counts, tiles[E+1] the same of their row tiles of kGrpBM, perm[q] the pair at sorted position q. Pairs
+// exclusive prefix of the per-expert counts, tiles[E+1] the same of their row tiles of bm rows (128 or
+// 256), perm[q] the pair at sorted position q. Pairs
 // whose expert id lies outside [0, E) are left out. The two prefixes are one wave's scan (four
 // experts a lane); a thread's ids of a pass are requested together. The order within an expert
 // follows the LDS atomics: every GEMM row is computed on its own, so it changes no result.
 constexpr int kSortThreads = 1024;
 __global__ void __launch_bounds__(kSortThreads) moe_sort_kernel(const int* __restrict__ idx, int n, int E,
-                                                                int* __restrict__ off, int* __restrict__ tiles,
+                                                                int bm, int* __restrict__ off, int* __restrict__ tiles,
                                                                 int* __restrict__ perm) {
   __shared__ int cnt[kMoeMaxE], cur[kMoeMaxE];
   const int tid = threadIdx.x;
@@ -382,7 +383,7 @@ __global__ void __launch_bounds__(kSortThreads) moe_sort_kernel(const int* __res
     for (int j = 0; j < 4; j++) {
       const int e = 4 * tid + j;
       c[j] = e < E ? cnt[e] : 0;
-      tl[j] = (c[j] + kGrpBM - 1) / kGrpBM;
+      tl[j] = (c[j] + bm - 1) / bm;
       cs += c[j];
       ts += tl[j];
     }
@@ -482,10 +483,10 @@ __global__ void __launch_bounds__(128) moe_combine_kernel(const f16* __restrict_
   }
 }
 
-// One grouped MFMA GEMM launch over the experts (gemm_kernel in grouped mode, tile kGrpBM x kGrpBN):
+// One grouped MFMA GEMM launch over the experts (gemm_kernel in grouped mode, tile BM x kGrpBN):
 // sorted rows [off[e], off[e+1]) of expert e times W + e * wstride_bytes. gather: A row q is
 // A row perm[q] / k (A has a_rows rows); scatter: C row q goes to C row perm[q].
-template <int EPI>
+template <int EPI, int BM, int WM, int S>
 int grouped_gemm(const f16* A, int lda, int a_rows, const f16* W, int64_t wstride_bytes, f16* C, int ldc, int N, int K,
                  const int* off, const int* tiles, const int* perm, int k, bool gather, bool scatter, int E,
                  int max_row_tiles, hipStream_t s) {
@@ -510,9 +511,9 @@ int grouped_gemm(const f16* A, int lda, int a_rows, const f16* W, int64_t wstrid
   g.grp_a_rows = a_rows;
   g.grp_gather = gather;
   g.grp_scatter = scatter;
-  auto fn = gemm_kernel<kGrpBM, kGrpBN, kGrpWM, kGrpWN, kGrpStages, EPI, false, true, kGrpBK>;
-  const size_t lds = std::max((size_t)kGrpStages * (kGrpBM + kGrpBN) * kGrpBK * 2, gemm_stage_bytes(kGrpBM, kGrpBN));
-  constexpr int threads = 64 * kGrpWM * kGrpWN;
+  auto fn = gemm_kernel<BM, kGrpBN, WM, kGrpWN, S, EPI, false, true, kGrpBK>;
+  const size_t lds = std::max((size_t)S * (BM + kGrpBN) * kGrpBK * 2, gemm_stage_bytes(BM, kGrpBN));
+  constexpr int threads = 64 * WM * kGrpWN;
   if (hi_blocks_per_cu(reinterpret_cast<const void*>(fn), threads, lds) <= 0) HI_FAIL("moe: grouped GEMM does not fit");
   const int tiles_n = (N + kGrpBN - 1) / kGrpBN;
   hipLaunchKernelGGL(fn, dim3(max_row_tiles * tiles_n), dim3(threads), lds, s, g);
@@ -526,8 +527,8 @@ size_t al256(size_t b) { return (b + 255) / 256 * 256; }
 int gemv_max() { return hi_gemv_max_rows(); }
 
 // The expert workspace (hi_moe_work_bytes), each piece on a 256-byte boundary. The first
-// kMoeBarBytes (at a fixed offset, whatever M) hold the one-token launch's arrival counters and the
-// grouped router's arrival counter; then perm [n], off and tiles [E+1] int, y [n, H] (pair order)
+// kMoeBarBytes (at a fixed offset, whatever M) hold the one-token launch's arrival counters, which no
+// other launch uses; then perm [n], off and tiles [E+1] int, y [n, H] (pair order)
 // and act [n, I] fp16 (sorted order on the grouped path, pair order on the GEMV path).
 constexpr int kMoeBarStride = 64;                 // words between two arrival counters (256 bytes)
 constexpr size_t kMoeBarBytes = 9 * 256;          // 8 counters, then the 8 expected totals
@@ -548,20 +549,39 @@ MoeWork moe_work(void* work, int n, int E, int H) {
   return m;
 }
 
-// The grouped path after the sort (perm / off / tiles in wk): gate/up + SwiGLU on the rows of xn
-// gathered by the tile DMA (act in sorted order), down scattered to pair order (y), the combine.
+// Row tile of the grouped GEMMs: 256 rows where the experts average 128 rows or more and 256-row tiles
+// still give every CU a block in both GEMMs. An expert of 129-256 rows is then one tile, its weights
+// streamed once, instead of two that are 30 % padding; a smaller grid would leave CUs idle. Measured,
+// whole layer, 128-row tiles -> 256: 32 experts, top 8, H 1024, I 512: 512 tokens 68.2 -> 62.9 us, 700
+// 75.7 -> 71.3, 2048 157.8 -> 148.0; 64 experts, top 6, H 2048, I 768: 1400 tokens 268.7 -> 249.8, 2048
+// 344.6 -> 287.3. What bounds the GEMMs is their ring's start and end (16 and 8 K tiles) per round.
+bool moe_tall(int n, int E, int H, int I, int cus) {
+  const int row_tiles = std::max(E, n / kGrpTallBM), tiles_n = (std::min(2 * I, H) + kGrpBN - 1) / kGrpBN;
+  return n / 128 >= E && (int64_t)row_tiles * tiles_n >= cus;
+}
+
+// The grouped path: the sort (perm / off / tiles in wk), gate/up + SwiGLU on the rows of xn gathered by
+// the tile DMA (act in sorted order), down scattered to pair order (y), the combine.
 int moe_grouped(const f16* xn, int ldxn, const f16* Wgu, const f16* Wd, const int* idx, const float* w, int M, int E,
                 int k, int H, int I, int flags, float scale, f16* x, int ldx, const MoeWork& wk, hipStream_t st) {
+  const HiDevice* d = hi_device();
+  if (!d) return -2;
   const int n = M * k;
   // the tile DMA addresses xn's gathered rows, and act's and y's rows, at 32-bit byte offsets
   if ((int64_t)M * ldxn * 2 >= INT32_MAX || (int64_t)n * (H > I ? H : I) * 2 >= INT32_MAX)
     HI_FAIL("moe: %d rows too many for the grouped path's 32-bit offsets", M);
-  const int max_row_tiles = (n + kGrpBM - 1) / kGrpBM + E;  // each expert adds at most one partial tile
-  if (int r = grouped_gemm<2>(xn, ldxn, M, Wgu, (int64_t)2 * I * H * 2, wk.act, I, 2 * I, H, wk.off, wk.tiles, wk.perm,
-                              k, true, false, E, max_row_tiles, st))
+  const bool tall = moe_tall(n, E, H, I, d->cus);
+  const int bm = tall ? kGrpTallBM : kGrpBM;
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kSortThreads), 0, st, idx, n, E, bm, wk.off, wk.tiles, wk.perm);
+  HI_TRY(hipGetLastError());
+  const int max_row_tiles = (n + bm - 1) / bm + E;  // each expert adds at most one partial tile
+  const auto gu = tall ? grouped_gemm<2, kGrpTallBM, kGrpTallWM, kGrpTallStages> : grouped_gemm<2, kGrpBM, kGrpWM, kGrpStages>;
+  const auto down = tall ? grouped_gemm<0, kGrpTallBM, kGrpTallWM, kGrpTallStages> : grouped_gemm<0, kGrpBM, kGrpWM, kGrpStages>;
+  if (int r = gu(xn, ldxn, M, Wgu, (int64_t)2 * I * H * 2, wk.act, I, 2 * I, H, wk.off, wk.tiles, wk.perm, k, true, false,
+                 E, max_row_tiles, st))
     return r;
-  if (int r = grouped_gemm<0>(wk.act, I, n, Wd, (int64_t)H * I * 2, wk.y, H, H, I, wk.off, wk.tiles, wk.perm, 1, false,
-                              true, E, max_row_tiles, st))
+  if (int r = down(wk.act, I, n, Wd, (int64_t)H * I * 2, wk.y, H, H, I, wk.off, wk.tiles, wk.perm, 1, false, true, E,
+                   max_row_tiles, st))
     return r;
   const auto comb = k <= 4 ? moe_combine_kernel<4> : k <= 8 ? moe_combine_kernel<8> : moe_combine_kernel<16>;
   hipLaunchKernelGGL(comb, dim3(M), dim3(128), 0, st, wk.y, idx, w, k, E, H, flags, scale, x, (int64_t)ldx);
@@ -939,8 +959,6 @@ HI_EXPORT int hi_moe_experts(const void* xn, int ldxn, const void* wgu, const vo
     HI_TRY(hipGetLastError());
     return moe_down_launch(wk.act, Wd, idx, w, M, k, E, H, I, flags, scale, x, ldx, st);
   }
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kSortThreads), 0, st, idx, n, E, wk.off, wk.tiles, wk.perm);
-  HI_TRY(hipGetLastError());
   return moe_grouped((const f16*)xn, ldxn, Wgu, Wd, idx, w, M, E, k, H, I, flags, scale, (f16*)x, ldx, wk, st);
 }
 
@@ -973,8 +991,6 @@ HI_EXPORT int hi_moe_route_experts(const void* xn, int ldxn, const void* Wr, con
   const MoeWork wk = moe_work(work, n, E, H);
   if (M > gemv_max()) {  // the router, then the grouped experts (sort, two GEMMs, combine)
     if (int r = hi_moe_router(xn, ldxn, Wr, M, E, H, k, flags, idx, w, s)) return r;
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kSortThreads), 0, st, idx, n, E, wk.off, wk.tiles, wk.perm);
-    HI_TRY(hipGetLastError());
     return moe_grouped((const f16*)xn, ldxn, (const f16*)wgu, (const f16*)wdown, idx, w, M, E, k, H, I, flags, scale,
                        (f16*)x, ldx, wk, st);
   }

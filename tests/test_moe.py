@@ -108,6 +108,28 @@ def test_moe_grouped_path_graph_replay(hi, O):
         hi.moe_experts(xn_d, wgu_d, wdn_d, idx_d, w_d, cuda(x0), flags, 0.22, 2)  # eager work between replays
 
 
+@pytest.mark.parametrize("H,I", [(1024, 512), (1056, 544)])
+def test_moe_grouped_tall_tiles_bit_identical(hi, H, I):
+    """128 rows per expert on average take the 256-row tiles, whose sums run in the 128-row tiles'
+    order: experts of no row, of one, and of either tile's edges, against calls of 400 tokens (the
+    128-row tiles, checked against the oracle above), bit for bit."""
+    r = rng(440 + H)
+    E, flags = 32, 1
+    counts = [0, 1, 127, 128, 129, 255, 256, 257, 511, 512, 513] + [90] * 21
+    ids = np.concatenate([np.full(c, e) for e, c in enumerate(counts)] + [[-1, E]]).astype(np.int32)
+    r.shuffle(ids)
+    M = len(ids)
+    assert (M - 2) // 128 >= E
+    wgu, wdn = cuda(rn(r, E, 2 * I, H, s=0.02)), cuda(rn(r, E, H, I, s=0.02))
+    xn, x0, idx = cuda(rn(r, M, H)), cuda(rn(r, M, H)), cuda(ids[:, None])
+    w = cuda(r.random((M, 1)).astype(np.float32))
+    got = host(hi.moe_experts(xn, wgu, wdn, idx, w, x0.clone(), flags, 0.22, 2))
+    for a in range(0, M, 400):
+        b = slice(a, min(a + 400, M))
+        ref = host(hi.moe_experts(xn[b], wgu, wdn, idx[b], w[b], x0[b].clone(), flags, 0.22, 2))
+        assert np.array_equal(got[b].view(np.uint16), ref.view(np.uint16)), f"rows {a}.."
+
+
 def test_moe_out_of_range_expert_ids_contribute_nothing(hi, O):
     r = rng(430)
     E, k, H, I, flags = 8, 2, 512, 256, 1
