@@ -549,15 +549,17 @@ MoeWork moe_work(void* work, int n, int E, int H) {
   return m;
 }
 
-// Row tile of the grouped GEMMs: 256 rows where the experts average 128 rows or more and 256-row tiles
+// Row tile of the grouped GEMMs: 256 rows where the experts average 112 rows or more and 256-row tiles
 // still give every CU a block in both GEMMs. An expert of 129-256 rows is then one tile, its weights
 // streamed once, instead of two that are 30 % padding; a smaller grid would leave CUs idle. Measured,
 // whole layer, 128-row tiles -> 256: 32 experts, top 8, H 1024, I 512: 512 tokens 68.2 -> 62.9 us, 700
 // 75.7 -> 71.3, 2048 157.8 -> 148.0; 64 experts, top 6, H 2048, I 768: 1400 tokens 268.7 -> 249.8, 2048
-// 344.6 -> 287.3. What bounds the GEMMs is their ring's start and end (16 and 8 K tiles) per round.
+// 344.6 -> 287.3. The line: evenly routed experts of 100 rows on average all fit 128 rows and
+// are slower in 256 (400 tokens 48.8 -> 54.4); of 120 some do not, and their second tiles start another
+// round (448 tokens 68.1 -> 58.3, 480 66.9 -> 56.4). What bounds the GEMMs is their ring's start and end (16 and 8 K tiles) per round.
 bool moe_tall(int n, int E, int H, int I, int cus) {
   const int row_tiles = std::max(E, n / kGrpTallBM), tiles_n = (std::min(2 * I, H) + kGrpBN - 1) / kGrpBN;
-  return n / 128 >= E && (int64_t)row_tiles * tiles_n >= cus;
+  return n / 112 >= E && (int64_t)row_tiles * tiles_n >= cus;
 }
 
 // The grouped path: the sort (perm / off / tiles in wk), gate/up + SwiGLU on the rows of xn gathered by
