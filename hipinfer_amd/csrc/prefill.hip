@@ -37,8 +37,9 @@
 //    blocks within each 16-lane group; O^T keeps the lane -> query row map, so the per-row
 //    rescale by exp2(m_old - m_new) is per lane;
 //  * causal mask on absolute positions (row t at p0 + t sees keys 0..p0+t): only the block's last
-//    one or two tiles (and an odd one before them) carry the mask arithmetic; cache rows past the
-//    block's last key read as zeros (the DMA's buffer range ends there);
+//    one or two tiles (and an odd one before them) carry the mask arithmetic, and a wave leaves out
+//    the key halves wholly above its rows' diagonal; cache rows past the block's last key read as
+//    zeros (the DMA's buffer range ends there);
 //  * blocks run the longest query tiles (the most keys) first, across all heads.
 #include <type_traits>
 
@@ -416,12 +417,36 @@ __global__ void __launch_bounds__(128 * RG)
     tile(kEven, no, yes, t, sa, sb);
     tile(kOdd, no, yes, t + 1, sb, sa);
   }
+  // The other tiles may hold masked keys. A wave leaves out a tile whose keys (its half) lie wholly past
+  // its rows' diagonal or the block's last key, as it does every later one, but for its share of the
+  // DMA and the barrier: their weights are 0, but 0 times an infinity or NaN in a later row's V is not.
+  auto live = [&](int t) {
+    const int k0 = t * kFpBKV + kFpKPW * kh;
+    return k0 <= p0 + qw + 31 && k0 < kv_end;
+  };
   for (; t + 1 < nt; t++) {  // an odd full tile, the first of two tiles on the diagonal
-    tile(t & 1, yes, yes, t, sa, sb);
-    sa[0] = sb[0];
-    sa[1] = sb[1];
+    if (live(t)) {
+      tile(t & 1, yes, yes, t, sa, sb);
+      sa[0] = sb[0];
+      sa[1] = sb[1];
+    } else {
+      wait_lgkm0();
+      wait_vmcnt<0>();
+      barrier_no_fence();
+#pragma unroll
+      for (int i = 0; i < IPW; i++) {
+        issue_k(i, t & 1);
+        issue_v(i, (t & 1) ^ 1);
+      }
+    }
   }
-  tile(t & 1, yes, no, t, sa, sb);
+  if (live(t)) {
+    tile(t & 1, yes, no, t, sa, sb);
+  } else {
+    wait_lgkm0();
+    wait_vmcnt<0>();
+    barrier_no_fence();
+  }
 
   pv(vl, pl);
 

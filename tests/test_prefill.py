@@ -148,6 +148,33 @@ def test_flash_prefill_row_block_rule(hi, O, D, Hq, T, p0):
         check(f"flash prefill lse row {t}", host(lse)[:, t:t + 1], ref_lse, 1e-4, 1e-5)
 
 
+@pytest.mark.parametrize("D,Hq,T,p0", [(128, 2, 200, 0), (128, 2, 200, 20), (64, 2, 200, 20), (128, 32, 600, 0),
+                                       (128, 32, 600, 101), (64, 32, 1100, 0), (64, 32, 600, 700)])
+def test_flash_prefill_non_finite_later_rows(hi, D, Hq, T, p0):
+    """A wave leaves out the 64-key halves of a 128-key tile that lie wholly past its 32 rows' diagonal, so
+    infinities and NaN in such a key's K and V rows change nothing for them, in either block height (the
+    first three shapes take 64-row blocks, the others 128): out and lse as with finite rows, bit for bit."""
+    r = rng(1310 + D + T + p0)
+    Hkv, S = 2, p0 + T
+    kc = cuda(r.standard_normal((Hkv, S, D)).astype(np.float16))
+    vc = cuda(r.standard_normal((Hkv, S, D)).astype(np.float16))
+    q = cuda(r.standard_normal((T, Hq * D)).astype(np.float16))
+    out, lse = (host(a) for a in hi.flash_prefill_lse(q, kc, vc, T, p0, Hq, Hkv))
+    assert np.isfinite(out).all() and np.isfinite(lse).all()
+    last_key = p0 + np.arange(T) // 32 * 32 + 31  # the last key that any row of row t's wave can see
+    checked = 0
+    for bad in sorted({60, 64, 127, 128, 191, T // 2, T - 1}):
+        kb, vb = kc.clone(), vc.clone()
+        for a, v in ((kb, float("-inf")), (vb, float("inf")), (vb, float("nan"))):
+            a[:, p0 + bad, (0 if v == v else 1)::2] = v
+        got, got_lse = (host(a) for a in hi.flash_prefill_lse(q, kb, vb, T, p0, Hq, Hkv))
+        rows = last_key < (p0 + bad) // 64 * 64
+        checked += rows.any()
+        assert np.array_equal(got[rows].view(np.uint16), out[rows].view(np.uint16)), f"key {p0 + bad}"
+        assert np.array_equal(got_lse[:, rows], lse[:, rows]), f"lse, key {p0 + bad}"
+    assert checked >= 3
+
+
 def test_flash_prefill_fused_qkv_rows_and_lse(hi, O):
     """q read in place from the rows of a fused qkv buffer (ldq = (Hq + 2 Hkv) D), output into a
     padded buffer (ldo > Hq D, the padding untouched), lse against the oracle's."""
