@@ -177,9 +177,11 @@ __global__ void __launch_bounds__(NWV * 64, 3) decode_attn_kernel(
         if (LAST && t0 + 8 * fk + k >= end) p[k] = -__builtin_huge_valf();
         mx = fmaxf(mx, p[k]);
       }
-      const float mn = fmaxf(m, rows_reduce<true>(mx));  // finite: every tile has a valid key
-      const float alpha = exp2f(m - mn);                 // 0 on the first tile (m = -inf)
-      m = mn;
+      const float m_old = m;
+      m = fmaxf(m, rows_reduce<true>(mx));
+      // -inf while every logit so far is (an infinity in K or q): their weights are 0
+      const float mn = m == -__builtin_huge_valf() ? 0.f : m;
+      const float alpha = exp2f(m_old - mn);  // 0 on the first tile (m = -inf)
       float ps = 0.f;
       f16x8 pf;
 #pragma unroll

@@ -89,6 +89,29 @@ def test_decode_attn_tile_and_split_edges(hi, O, D, Hkv, G, B):
         check(f"decode attn D={D} G={G} B={B} lens={lens[:4]}", got, O.decode_attn(q, kc, vc, pos, Hq, Hkv), 2e-3, 1e-2)
 
 
+@pytest.mark.parametrize("D,Hkv,G", [(64, 4, 8), (128, 8, 4)], ids=["D64-G8", "D128-G4"])
+@pytest.mark.parametrize("B,n", [(1, 64), (1, 700), (3, 300), (70, 200)])
+def test_decode_attn_minus_infinite_logits(hi, D, Hkv, G, B, n):
+    """Keys whose logit is -inf have weight 0, also where they are every key a wave sees first (its first 32,
+    or its last, partly filled tile): the result is that of the other keys, in float64 on the CPU."""
+    r = rng(680 + B + n)
+    Hq = Hkv * G
+    q = r.standard_normal((B, Hq * D)).astype(np.float16)
+    q.reshape(B, Hq, D)[:, :, 5] = 1.0 + r.random((B, Hq))
+    kc = r.standard_normal((B, Hkv, n, D)).astype(np.float16)
+    vc = r.standard_normal((B, Hkv, n, D)).astype(np.float16)
+    pos = np.full(B, n - 1, np.int32)
+    for lo, hi_ in ((0, 32), (n - n % 32 if n % 32 else n - 32, n), (17, 60)):
+        kb = kc.copy()
+        kb[:, :, lo:hi_, 5] = -np.inf
+        got = host(hi.decode_attn(cuda(q), cuda(kb), cuda(vc), cuda(pos), Hq, Hkv))
+        keep = np.r_[0:lo, hi_:n]
+        s = np.einsum("bhgd,bhkd->bhgk", q.reshape(B, Hkv, G, D).astype(np.float64), kc[:, :, keep].astype(np.float64))
+        p = np.exp(s / np.sqrt(D) - (s / np.sqrt(D)).max(-1, keepdims=True))
+        ref = np.einsum("bhgk,bhkd->bhgd", p, vc[:, :, keep].astype(np.float64)) / p.sum(-1)[..., None]
+        check(f"decode attn D={D} B={B} n={n} keys {lo}..{hi_} at -inf", got, ref.reshape(B, Hq * D), 2e-3, 1e-2)
+
+
 def test_decode_work_reuse(hi, O):
     """One zeroed work buffer for launches of decreasing and increasing batch: the split counters
     must be left zeroed and never land in a larger launch's partials. One kv head per sequence
