@@ -66,9 +66,8 @@ __device__ __forceinline__ float rows_reduce(float v) {
 // one per 256 keys, but down to 128 keys a split while there are at most
 // 16 (what the merge requests in one round): shorter waves finish sooner, and more splits cost more
 // in the merge (one sequence of 4001 keys, 32/8 heads: 16 splits 10.8 us, 32 splits 12.5; of 2500: 16
-// 9.5, 10 9.9). Beyond them only for runs over 1024 keys, which would end a ragged batch late (30
-// sequences of 500 to 4000: 73 -> 71 us); at 512 keys a uniform batch of 64 x 1000 leaves a part-filled
-// last round (49.8 -> 54.7).
+// 9.5, 10 9.9). Beyond S1, where the launch has them (decode_splits_max), only for runs over 1024 keys,
+// which would end a ragged batch late.
 __device__ __forceinline__ int splits_used(int len, int S, int S1) {
   return max(min(S1, max((len + 255) / 256, min(16, (len + 127) / 128))), min(S, (len + 1023) / 1024));
 }
@@ -322,6 +321,23 @@ __global__ void __launch_bounds__(NWV * 64, 3) decode_attn_kernel(
 // work buffer's 64.
 int decode_splits(int B, int Hkv, int cus) { return min((2 * cus + B * Hkv - 1) / (B * Hkv), kDecodeMaxSplits); }
 
+// Splits per pair that a launch has for its long runs (splits_used): 2 S1, or S1 where more would be spread
+// worse over the CUs. A batch may be uniform, all of its pairs then take S1 + 1 splits at once: S1 blocks
+// a pair that are a whole number for every CU stay that, and so do those whose last layer over the CUs
+// would be left emptier by more than a sixteenth of all layers. At S1 = 1 a second split also brings the
+// partials and their merge, and a part-filled second round of blocks (a CU holds 3 at D = 128). Measured
+// with 32/8 heads of 128, S1 alone / up to 2 S1, us: 64 x 1025 keys 49.6 / 55.1, 64 x 2000 94.1 / 100.5,
+// 120 x 1025 91.6 / 101.8, 16 x 4097 52.8 / 57.1, 44 x 2049 70.9 / 76.7; 24 x 3073 66.0 / 60.6, 52 x 2049
+// 89.5 / 85.8, 30 of 500 to 4000 70.0 / 66.0, 24 of 576 to 4608 68.8 / 54.5. It reads no lengths: a
+// sequence's sums do not depend on its neighbours'.
+int decode_splits_max(int B, int Hkv, int S1, int cus) {
+  const int n0 = B * Hkv * S1, n1 = n0 + B * Hkv;  // blocks
+  const int l0 = (n0 + cus - 1) / cus, l1 = (n1 + cus - 1) / cus;  // layers of one block a CU
+  // n0 / (l0 cus) and n1 / (l1 cus) are the shares of the layers that are filled
+  const bool worse = S1 == 1 || n0 % cus == 0 || 16 * ((int64_t)n0 * l1 - (int64_t)n1 * l0) > (int64_t)l0 * l1 * cus;
+  return worse ? S1 : min(2 * S1, kDecodeMaxSplits);
+}
+
 template <int D>
 int decode_attn_d(int G, dim3 grid, hipStream_t s, const f16* q, int ldq, const f16* kc, const f16* vc, int max_seq,
                   int Hkv, const int* pos, float* part, int* counters, int S, int S1, f16* out, int ldo, float sl2,
@@ -476,7 +492,8 @@ static int decode_attn_run(const void* q, int ldq, const void* kc, const void* v
     HI_FAIL("%s: q, kc and vc must be 16-byte aligned and ldq a multiple of 8", who);
   if (ldq < Hq * D || ldo < Hq * D) HI_FAIL("%s: ldq %d / ldo %d < Hq * D = %d", who, ldq, ldo, Hq * D);
   // one sequence (kv_slot >= 0): a batch of one's split count, so every row matches that decode
-  const int S1 = decode_splits(kv_slot >= 0 ? 1 : B, Hkv, d->cus), S = min(2 * S1, kDecodeMaxSplits);
+  const int Bs = kv_slot >= 0 ? 1 : B;
+  const int S1 = decode_splits(Bs, Hkv, d->cus), S = decode_splits_max(Bs, Hkv, S1, d->cus);
   const float sl2 = 1.4426950408889634f / sqrtf((float)D);
   const dim3 grid(S * Hkv * B);  // split-major: (split, sequence, kv head)
   int* counters = (int*)work;

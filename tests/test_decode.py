@@ -112,6 +112,31 @@ def test_decode_attn_minus_infinite_logits(hi, D, Hkv, G, B, n):
         check(f"decode attn D={D} B={B} n={n} keys {lo}..{hi_} at -inf", got, ref.reshape(B, Hq * D), 2e-3, 1e-2)
 
 
+@pytest.mark.parametrize("B,Hkv,splits", [(512, 1, 1), (64, 8, 1), (44, 8, 2), (24, 8, 4)])
+def test_decode_attn_splits_of_long_uniform_batches(hi, B, Hkv, splits):
+    """Splits per (sequence, kv head) pair of a batch of equal lengths, read from the partial results in the work
+    buffer. Pairs that alone give every CU two blocks stay one split at every length (a second would be a
+    part-filled second round of blocks: the time of 64 x 1025 keys went up by a tenth over 64 x 1024), and 44 x
+    8 stay two; 24 x 8 take a fourth over 3072 keys. On 256 CUs."""
+    import torch
+    if hi.lib.hi_device_cus() != 256:
+        pytest.skip("the counts are those of 256 CUs")
+    D, first = 64, 1024 * max(1, splits - (splits > 2)) + 1
+    for n in (first - 1, first, first + 900):
+        g = torch.Generator(device="cuda").manual_seed(n)
+        kc, vc = (torch.randn(B, Hkv, n, D, device="cuda", generator=g).half() for _ in range(2))
+        q = torch.randn(B, Hkv * D, device="cuda", generator=g).half()
+        pos = torch.full((B,), n - 1, dtype=torch.int32, device="cuda")
+        work = torch.zeros(hi.lib.hi_decode_work_bytes(B, Hkv, Hkv, D), dtype=torch.uint8, device="cuda")
+        got = hi.decode_attn(q, kc, vc, pos, Hkv, Hkv, work=work).float().view(B, Hkv, D)
+        sums = work[4096 * 4:].view(torch.float32).view(B, Hkv, 64, D + 2)[..., D + 1]
+        used = splits - (splits > 2 and n <= 3072)
+        assert ((sums != 0).sum(-1) == (used if used > 1 else 0)).all(), f"splits at {n} keys"
+        s = (kc.float() * q.float().view(B, Hkv, 1, D)).sum(-1) / D ** 0.5
+        ref = (torch.softmax(s, -1)[..., None] * vc.float()).sum(2)
+        check(f"decode attn {B} x {n}", host(got), host(ref), 2e-3, 1e-2)
+
+
 def test_decode_work_reuse(hi, O):
     """One zeroed work buffer for launches of decreasing and increasing batch: the split counters
     must be left zeroed and never land in a larger launch's partials. One kv head per sequence
