@@ -66,9 +66,11 @@ __device__ __forceinline__ float rows_reduce(float v) {
 // one per 256 keys, but down to 128 keys a split while there are at most
 // 16 (what the merge requests in one round): shorter waves finish sooner, and more splits cost more
 // in the merge (one sequence of 4001 keys, 32/8 heads: 16 splits 10.8 us, 32 splits 12.5; of 2500: 16
-// 9.5, 10 9.9). Beyond S1, where the launch has them (decode_splits_max), only for runs over 1024 keys,
-// which would end a ragged batch late.
+// 9.5, 10 9.9). Up to 256 keys one split, which has no partials and no merge (200 keys, two splits / one, us:
+// one sequence 7.3 / 5.8, 8 of them 8.6 / 6.2, 24 10.5 / 6.9). Beyond S1, where the launch has them
+// (decode_splits_max), only for runs over 1024 keys, which would end a ragged batch late.
 __device__ __forceinline__ int splits_used(int len, int S, int S1) {
+  if (len <= 256) return 1;
   return max(min(S1, max((len + 255) / 256, min(16, (len + 127) / 128))), min(S, (len + 1023) / 1024));
 }
 

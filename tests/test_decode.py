@@ -112,29 +112,42 @@ def test_decode_attn_minus_infinite_logits(hi, D, Hkv, G, B, n):
         check(f"decode attn D={D} B={B} n={n} keys {lo}..{hi_} at -inf", got, ref.reshape(B, Hq * D), 2e-3, 1e-2)
 
 
-@pytest.mark.parametrize("B,Hkv,splits", [(512, 1, 1), (64, 8, 1), (44, 8, 2), (24, 8, 4)])
-def test_decode_attn_splits_of_long_uniform_batches(hi, B, Hkv, splits):
-    """Splits per (sequence, kv head) pair of a batch of equal lengths, read from the partial results in the work
-    buffer. Pairs that alone give every CU two blocks stay one split at every length (a second would be a
-    part-filled second round of blocks: the time of 64 x 1025 keys went up by a tenth over 64 x 1024), and 44 x
-    8 stay two; 24 x 8 take a fourth over 3072 keys. On 256 CUs."""
+def splits_run(hi, B, Hkv, n, D=64):
+    """Splits per (sequence, kv head) pair that a batch of B sequences of n keys ran, counted in the partial
+    results left in the work buffer (none for one split); the output is checked on the way."""
     import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    kc, vc = (torch.randn(B, Hkv, n, D, device="cuda", generator=g).half() for _ in range(2))
+    q = torch.randn(B, Hkv * D, device="cuda", generator=g).half()
+    pos = torch.full((B,), n - 1, dtype=torch.int32, device="cuda")
+    work = torch.zeros(hi.lib.hi_decode_work_bytes(B, Hkv, Hkv, D), dtype=torch.uint8, device="cuda")
+    got = hi.decode_attn(q, kc, vc, pos, Hkv, Hkv, work=work).float().view(B, Hkv, D)
+    s = (kc.float() * q.float().view(B, Hkv, 1, D)).sum(-1) / D ** 0.5
+    ref = (torch.softmax(s, -1)[..., None] * vc.float()).sum(2)
+    check(f"decode attn {B} x {n}", host(got), host(ref), 2e-3, 1e-2)
+    sums = work[4096 * 4:].view(torch.float32).view(B, Hkv, 64, D + 2)[..., D + 1]
+    count = (sums != 0).sum(-1)
+    assert (count == count[0, 0]).all()
+    return max(1, int(count[0, 0]))
+
+
+@pytest.mark.parametrize("B,Hkv,n,splits", [
+    (512, 1, 1024, 1), (512, 1, 1025, 1), (512, 1, 1900, 1), (64, 8, 1025, 1), (64, 8, 1900, 1),
+    (44, 8, 2048, 2), (44, 8, 2049, 2), (44, 8, 2900, 2), (24, 8, 3072, 3), (24, 8, 3073, 4)])
+def test_decode_attn_splits_of_long_uniform_batches(hi, B, Hkv, n, splits):
+    """Pairs that alone give every CU two blocks stay one split at every length (a second would be a part-filled
+    second round of blocks: the time of 64 x 1025 keys went up by a tenth over 64 x 1024), and 44 x 8 stay
+    two; 24 x 8 take a fourth over 3072 keys. On 256 CUs."""
     if hi.lib.hi_device_cus() != 256:
         pytest.skip("the counts are those of 256 CUs")
-    D, first = 64, 1024 * max(1, splits - (splits > 2)) + 1
-    for n in (first - 1, first, first + 900):
-        g = torch.Generator(device="cuda").manual_seed(n)
-        kc, vc = (torch.randn(B, Hkv, n, D, device="cuda", generator=g).half() for _ in range(2))
-        q = torch.randn(B, Hkv * D, device="cuda", generator=g).half()
-        pos = torch.full((B,), n - 1, dtype=torch.int32, device="cuda")
-        work = torch.zeros(hi.lib.hi_decode_work_bytes(B, Hkv, Hkv, D), dtype=torch.uint8, device="cuda")
-        got = hi.decode_attn(q, kc, vc, pos, Hkv, Hkv, work=work).float().view(B, Hkv, D)
-        sums = work[4096 * 4:].view(torch.float32).view(B, Hkv, 64, D + 2)[..., D + 1]
-        used = splits - (splits > 2 and n <= 3072)
-        assert ((sums != 0).sum(-1) == (used if used > 1 else 0)).all(), f"splits at {n} keys"
-        s = (kc.float() * q.float().view(B, Hkv, 1, D)).sum(-1) / D ** 0.5
-        ref = (torch.softmax(s, -1)[..., None] * vc.float()).sum(2)
-        check(f"decode attn {B} x {n}", host(got), host(ref), 2e-3, 1e-2)
+    assert splits_run(hi, B, Hkv, n) == splits
+
+
+@pytest.mark.parametrize("B", [1, 5, 24])
+def test_decode_attn_one_split_up_to_256_keys(hi, B):
+    """A short context needs no merge: two splits of 100 keys took a quarter longer than one of 200."""
+    assert [splits_run(hi, B, 8, n) for n in (1, 129, 200, 256)] == [1] * 4
+    assert splits_run(hi, B, 8, 257) > 1
 
 
 def test_decode_work_reuse(hi, O):
