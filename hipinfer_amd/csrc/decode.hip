@@ -62,8 +62,8 @@ __device__ __forceinline__ float rows_reduce(float v) {
   return v;
 }
 
-// Splits in use for `len` keys when a launch has S per pair and S1 give every CU two blocks: of those,
-// one per 256 keys, but down to 128 keys a split while there are at most
+// Splits in use for `len` keys when a launch has S per pair, S1 of them to give every CU its two blocks (one of
+// 8 waves): of those, one per 256 keys, but down to 128 keys a split while there are at most
 // 16 (what the merge requests in one round): shorter waves finish sooner, and more splits cost more
 // in the merge (one sequence of 4001 keys, 32/8 heads: 16 splits 10.8 us, 32 splits 12.5; of 2500: 16
 // 9.5, 10 9.9). Up to 256 keys one split, which has no partials and no merge (200 keys, two splits / one, us:
@@ -323,6 +323,17 @@ __global__ void __launch_bounds__(NWV * 64, 3) decode_attn_kernel(
 // work buffer's 64.
 int decode_splits(int B, int Hkv, int cus) { return min((2 * cus + B * Hkv - 1) / (B * Hkv), kDecodeMaxSplits); }
 
+// Blocks of 8 waves where that is 16 or more (at most about an eighth as many pairs as CUs): a launch this
+// small is a chain of latencies, and a block of 256 keys is then one tile per wave (one sequence of
+// 2500 keys 9.45 -> 9.0 us, of 8000 14.8 -> 13.8, four of 700 to 800 at D = 64 8.1 -> 7.4); with more
+// pairs 4 waves balance better (40 sequences of 300 to 2400, 12/2 heads: 19.5 against 25.5). A CU holds one
+// such block at D = 128 (12 waves of 137 registers), so the launch has at most one for each: with two, the
+// lengths that use more than half of them run a part-filled second round (32/8 heads of 128, two / one, us: one
+// sequence of 12000 21.4 / 17.0, two of 6000 20.8 / 16.7, four of 2000 15.3 / 11.9, one of 32000 34.4 / 29.6; two
+// of 6000, 32/4 heads of 64, 10.5 / 10.4, of 20000 18.5 / 15.3).
+constexpr int kDaWideSplits = 16;
+int decode_splits_wide(int B, int Hkv, int cus) { return min(max(cus / (B * Hkv), 1), kDecodeMaxSplits); }
+
 // Splits per pair that a launch has for its long runs (splits_used): 2 S1, or S1 where more would be spread
 // worse over the CUs. A batch may be uniform, all of its pairs then take S1 + 1 splits at once: S1 blocks
 // a pair that are a whole number for every CU stay that, and so do those whose last layer over the CUs
@@ -342,13 +353,8 @@ int decode_splits_max(int B, int Hkv, int S1, int cus) {
 
 template <int D>
 int decode_attn_d(int G, dim3 grid, hipStream_t s, const f16* q, int ldq, const f16* kc, const f16* vc, int max_seq,
-                  int Hkv, const int* pos, float* part, int* counters, int S, int S1, f16* out, int ldo, float sl2,
-                  int kv_slot) {
-  // 8 waves where S1 is 16 or more (at most about an eighth as many pairs as CUs): a launch this
-  // small is a chain of latencies, and a block of 256 keys is then one tile per wave (one sequence of
-  // 2500 keys 9.45 -> 9.0 us, of 8000 14.8 -> 13.8, four of 700 to 800 at D = 64 8.1 -> 7.4); with more
-  // pairs 4 waves balance better (40 sequences of 300 to 2400, 12/2 heads: 19.5 against 25.5).
-  const bool wide = S1 >= 16;
+                  int Hkv, const int* pos, float* part, int* counters, int S, int S1, bool wide, f16* out, int ldo,
+                  float sl2, int kv_slot) {
 #define HI_DA(g)                                                                                              \
   case g:                                                                                                     \
     if (wide)                                                                                                 \
@@ -495,7 +501,10 @@ static int decode_attn_run(const void* q, int ldq, const void* kc, const void* v
   if (ldq < Hq * D || ldo < Hq * D) HI_FAIL("%s: ldq %d / ldo %d < Hq * D = %d", who, ldq, ldo, Hq * D);
   // one sequence (kv_slot >= 0): a batch of one's split count, so every row matches that decode
   const int Bs = kv_slot >= 0 ? 1 : B;
-  const int S1 = decode_splits(Bs, Hkv, d->cus), S = decode_splits_max(Bs, Hkv, S1, d->cus);
+  int S1 = decode_splits(Bs, Hkv, d->cus), S;
+  const bool wide = S1 >= kDaWideSplits;
+  if (wide) S = S1 = decode_splits_wide(Bs, Hkv, d->cus);
+  else S = decode_splits_max(Bs, Hkv, S1, d->cus);
   const float sl2 = 1.4426950408889634f / sqrtf((float)D);
   const dim3 grid(S * Hkv * B);  // split-major: (split, sequence, kv head)
   int* counters = (int*)work;
@@ -503,9 +512,9 @@ static int decode_attn_run(const void* q, int ldq, const void* kc, const void* v
   const hipStream_t st = (hipStream_t)s;
   if (D == 64)
     return decode_attn_d<64>(Hq / Hkv, grid, st, (const f16*)q, ldq, (const f16*)kc, (const f16*)vc, max_seq, Hkv, pos,
-                             part, counters, S, S1, (f16*)out, ldo, sl2, kv_slot);
+                             part, counters, S, S1, wide, (f16*)out, ldo, sl2, kv_slot);
   return decode_attn_d<128>(Hq / Hkv, grid, st, (const f16*)q, ldq, (const f16*)kc, (const f16*)vc, max_seq, Hkv, pos,
-                            part, counters, S, S1, (f16*)out, ldo, sl2, kv_slot);
+                            part, counters, S, S1, wide, (f16*)out, ldo, sl2, kv_slot);
 }
 
 // out[b, h*D : (h+1)*D] = softmax(q_h . K[0..pos[b]] / sqrt(D)) V for every query head h of

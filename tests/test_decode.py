@@ -150,6 +150,16 @@ def test_decode_attn_one_split_up_to_256_keys(hi, B):
     assert splits_run(hi, B, 8, 257) > 1
 
 
+@pytest.mark.parametrize("B,n,splits", [(1, 8192, 32), (1, 8193, 32), (1, 12000, 32), (2, 6000, 16), (3, 4000, 10),
+                                        (4, 2000, 8), (4, 20000, 8)])
+def test_decode_attn_8_wave_launch_has_one_block_per_cu(hi, B, n, splits):
+    """Launches of 8-wave blocks, of which a CU holds one: no more of them than CUs, at any length (8 kv heads;
+    on 256 CUs)."""
+    if hi.lib.hi_device_cus() != 256:
+        pytest.skip("the counts are those of 256 CUs")
+    assert splits_run(hi, B, 8, n) == splits
+
+
 def test_decode_work_reuse(hi, O):
     """One zeroed work buffer for launches of decreasing and increasing batch: the split counters
     must be left zeroed and never land in a larger launch's partials. One kv head per sequence
