@@ -143,8 +143,28 @@ __device__ __forceinline__ void sched_step() {
   for (; v < NV; v++) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
 }
 
-template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, bool GRP = false, int BK = 64, int KG = 1, int SB = S>
-__global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
+// Grouped mode: what a thread loads of the groups before anything else (thread e < grp_n its group's tile
+// start and first row, thread 0 also the totals).
+struct GrpLoad {
+  int tile, off, tiles_all, off_all;
+};
+__device__ __forceinline__ GrpLoad grp_load(const GemmArgs& g) {
+  GrpLoad l{};
+  const int tid = threadIdx.x;
+  if (tid < g.grp_n) {
+    l.tile = g.grp_tiles[tid];
+    l.off = g.grp_off[tid];
+  }
+  if (tid == 0) {
+    l.tiles_all = g.grp_tiles[g.grp_n];
+    l.off_all = g.grp_off[g.grp_n];
+  }
+  return l;
+}
+
+// groups(): the thread's GrpLoad (grouped mode only)
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, bool GRP, int BK, int KG, int SB, class Groups>
+__device__ __forceinline__ void gemm_body(GemmArgs g, [[maybe_unused]] Groups groups) {
   constexpr int TM = BM / WM, TN = BN / WN;          // wave tile
   constexpr int FM = TM / 32, FN = TN / 32;          // MFMA tiles per wave
   constexpr int A_ST = BM * BK;                      // halves per stage
@@ -206,24 +226,23 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
   if constexpr (GRP) {
     // find this block's group: grp_tiles[e] <= row tile < grp_tiles[e + 1] (the prefix is
     // non-decreasing, so e is the number of groups whose tiles start at or before the row tile,
-    // minus one); blocks past the last row tile (the grid is sized for the worst case) exit. Every
-    // thread loads one group's tile start and first row at once (thread 0 also the totals): one
-    // memory round trip, then one counting barrier.
+    // minus one); blocks past the last row tile (the grid is sized for the worst case) exit. The
+    // threads have loaded the groups at once (grp_load): one memory round trip, then one counting
+    // barrier.
     static_assert(64 * NW * KG >= kGemmMaxGroups, "one thread per group");
     __shared__ int s_tiles[kGemmMaxGroups + 1], s_off[kGemmMaxGroups + 1];
     const int E = g.grp_n, mt = blockIdx.x / tiles_n;
     tn = blockIdx.x - mt * tiles_n;
-    int te = 0;
+    const GrpLoad gl = groups();
     if (tid < E) {
-      te = g.grp_tiles[tid];
-      s_tiles[tid] = te;
-      s_off[tid] = g.grp_off[tid];
+      s_tiles[tid] = gl.tile;
+      s_off[tid] = gl.off;
     }
     if (tid == 0) {
-      s_tiles[E] = g.grp_tiles[E];
-      s_off[E] = g.grp_off[E];
+      s_tiles[E] = gl.tiles_all;
+      s_off[E] = gl.off_all;
     }
-    const int lo = __syncthreads_count(tid < E && te <= mt) - 1;
+    const int lo = __syncthreads_count(tid < E && gl.tile <= mt) - 1;
     if (mt >= s_tiles[E]) return;
     grp_r0 = s_off[lo];
     M = s_off[lo + 1] - grp_r0;
@@ -709,6 +728,24 @@ __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
   }
 }
 
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, bool GRP = false, int BK = 64, int KG = 1, int SB = S>
+__global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
+  gemm_body<BM, BN, WM, WN, S, EPI, Q8, GRP, BK, KG, SB>(g, [&] { return grp_load(g); });
+}
+
+// Grouped mode with the tile's shape chosen on the device, which knows the groups' sizes: BM x BN or, where
+// grp_tiles[grp_n + 1] is not 0, BN x BM (and WN x WM waves: the wave tile, the ring and the order of the sums
+// are the same). That word is loaded with the groups, so the choice costs no round trip of its own.
+template <int BM, int BN, int WM, int WN, int S, int EPI, int BK>
+__global__ void __launch_bounds__(64 * WM * WN) gemm_grp_kernel(GemmArgs g) {
+  const int turned = g.grp_tiles[g.grp_n + 1];
+  const GrpLoad gl = grp_load(g);
+  if (turned == 0)
+    gemm_body<BM, BN, WM, WN, S, EPI, false, true, BK, 1, S>(g, [&] { return gl; });
+  else
+    gemm_body<BN, BM, WN, WM, S, EPI, false, true, BK, 1, S>(g, [&] { return gl; });
+}
+
 // Split-K second pass: sum the fp32 partials [splits][M][N] in split order (deterministic) and run
 // the epilogue with the main kernel's rounding; each thread owns 4 consecutive output columns.
 template <int EPI>
@@ -793,7 +830,7 @@ constexpr bool gemm_cfg_fits(int c, bool q8, int K) {
 // 64 rows each), so each expert's weights are streamed once; a 64-row tile split most experts into
 // two row tiles, each streaming the same weights.
 constexpr int kGrpBM = 128, kGrpBN = 128, kGrpWM = 2, kGrpWN = 2, kGrpStages = 4, kGrpBK = 64;
-// Tall variant for experts of more than 128 rows (8 waves, three stages of 48 KB).
+// The big tiles for experts of more than 128 rows: 256 x 128 or 128 x 256 (8 waves, three stages of 48 KB).
 constexpr int kGrpTallBM = 256, kGrpTallWM = 4, kGrpTallStages = 3;
 // Ring stages of a config's A and W tiles. The 64-deep 256 x 256 and 256 x 192 tiles hold one more
 // stage for W than for A (in fp16, 256 x 256 fills the CU's 160 KB with it): with two stages of

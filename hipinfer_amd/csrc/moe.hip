@@ -349,16 +349,33 @@ __global__ void __launch_bounds__(kMoeWaves * 64) moe_gemv_down_kernel(const f16
 }
 
 // ------------------------------------------------------------------ grouped path
-// Counting sort of the n (token, slot) pairs by expert, by one block of kSortThreads: off[E+1] the
-// exclusive prefix of the per-expert counts, tiles[E+1] the same of their row tiles of bm rows (128 or
-// 256), perm[q] the pair at sorted position q. Pairs
+// Counting sort of the n (token, slot) pairs by expert, by one block of kSortThreads: off[0..E] the
+// exclusive prefix of the per-expert counts, tiles[0..E] the same of their row tiles of bm rows (128, or
+// 256), perm[q] the pair at sorted position q. With bm 256 the counts decide between the tiles 256 x 128
+// and 128 x 256 (big_tiles_turned), and tiles[E+1], behind the prefix, tells the GEMMs. Pairs
 // whose expert id lies outside [0, E) are left out. The two prefixes are one wave's scan (four
 // experts a lane); a thread's ids of a pass are requested together. The order within an expert
 // follows the LDS atomics: every GEMM row is computed on its own, so it changes no result.
 constexpr int kSortThreads = 1024;
+
+// Whether the big tiles should be 128 rows x 256 columns rather than 256 x 128, for experts that come to t256
+// and t128 row tiles: where the GEMMs' blocks (gate/up [2I, H], down [H, I]; one per CU) make less rounds of
+// them, a round taking its K tiles and about 8 for the ring's start and end. 256 rows stream an expert of
+// up to 256 once, but experts over 256 rows, as uneven routing makes them, bring a few row tiles of 256 and
+// with them a part-filled second round; 128 rows also waste less on them. 32 experts, top 8, H 1024, I 512,
+// experts chosen in proportion to 1 / sqrt(rank), 256 x 128 / 128 x 256 / 128 x 128 with 4 waves, us: 600 tokens
+// 71.5 / 53.6 / 62.1, 700 73.8 / 57.6 / 64.8, 64 experts, top 6, H 2048, I 768: 1400 tokens 228.9 / 221.0 / 231.1.
+__device__ bool big_tiles_turned(int t256, int t128, int H, int I, int cus) {
+  auto rounds = [&](int row_tiles, int bn, int N) { return (row_tiles * ((N + bn - 1) / bn) + cus - 1) / cus; };
+  auto cost = [&](int row_tiles, int bn) {
+    return rounds(row_tiles, bn, 2 * I) * (H / kGrpBK + 8) + rounds(row_tiles, bn, H) * (I / kGrpBK + 8);
+  };
+  return cost(t128, kGrpTallBM) < cost(t256, kGrpBN);
+}
+
 __global__ void __launch_bounds__(kSortThreads) moe_sort_kernel(const int* __restrict__ idx, int n, int E,
-                                                                int bm, int* __restrict__ off, int* __restrict__ tiles,
-                                                                int* __restrict__ perm) {
+                                                                int bm, int H, int I, int cus, int* __restrict__ off,
+                                                                int* __restrict__ tiles, int* __restrict__ perm) {
   __shared__ int cnt[kMoeMaxE], cur[kMoeMaxE];
   const int tid = threadIdx.x;
   constexpr int P = 4;  // ids a thread requests together
@@ -380,9 +397,20 @@ __global__ void __launch_bounds__(kSortThreads) moe_sort_kernel(const int* __res
     static_assert(kMoeMaxE <= 4 * 64, "four experts a lane");
     int c[4], tl[4], cs = 0, ts = 0;
 #pragma unroll
+    for (int j = 0; j < 4; j++) c[j] = 4 * tid + j < E ? cnt[4 * tid + j] : 0;
+    if (bm == kGrpTallBM) {
+      float t256 = 0.f, t128 = 0.f;  // row tiles (below 2^24: exact)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        t256 += (float)((c[j] + kGrpTallBM - 1) / kGrpTallBM);
+        t128 += (float)((c[j] + kGrpBN - 1) / kGrpBN);
+      }
+      const bool turned = big_tiles_turned((int)wave_sum(t256), (int)wave_sum(t128), H, I, cus);
+      if (turned) bm = kGrpBN;
+      if (tid == 0) tiles[E + 1] = turned;
+    }
+#pragma unroll
     for (int j = 0; j < 4; j++) {
-      const int e = 4 * tid + j;
-      c[j] = e < E ? cnt[e] : 0;
       tl[j] = (c[j] + bm - 1) / bm;
       cs += c[j];
       ts += tl[j];
@@ -483,13 +511,14 @@ __global__ void __launch_bounds__(128) moe_combine_kernel(const f16* __restrict_
   }
 }
 
-// One grouped MFMA GEMM launch over the experts (gemm_kernel in grouped mode, tile BM x kGrpBN):
-// sorted rows [off[e], off[e+1]) of expert e times W + e * wstride_bytes. gather: A row q is
-// A row perm[q] / k (A has a_rows rows); scatter: C row q goes to C row perm[q].
-template <int EPI, int BM, int WM, int S>
+// One grouped MFMA GEMM launch over the experts (gemm_kernel in grouped mode, tile kGrpBM x kGrpBN, or
+// with BIG gemm_grp_kernel, tile kGrpTallBM x kGrpBN or turned): sorted rows [off[e], off[e+1]) of expert e
+// times W + e * wstride_bytes, n rows in all. gather: A row q is A row perm[q] / k (A has a_rows rows);
+// scatter: C row q goes to C row perm[q].
+template <int EPI, bool BIG>
 int grouped_gemm(const f16* A, int lda, int a_rows, const f16* W, int64_t wstride_bytes, f16* C, int ldc, int N, int K,
                  const int* off, const int* tiles, const int* perm, int k, bool gather, bool scatter, int E,
-                 int max_row_tiles, hipStream_t s) {
+                 int n, hipStream_t s) {
   GemmArgs g{};
   g.A = A;
   g.lda = lda;
@@ -511,12 +540,18 @@ int grouped_gemm(const f16* A, int lda, int a_rows, const f16* W, int64_t wstrid
   g.grp_a_rows = a_rows;
   g.grp_gather = gather;
   g.grp_scatter = scatter;
-  auto fn = gemm_kernel<BM, kGrpBN, WM, kGrpWN, S, EPI, false, true, kGrpBK>;
-  const size_t lds = std::max((size_t)S * (BM + kGrpBN) * kGrpBK * 2, gemm_stage_bytes(BM, kGrpBN));
+  constexpr int BM = BIG ? kGrpTallBM : kGrpBM, WM = BIG ? kGrpTallWM : kGrpWM, S = BIG ? kGrpTallStages : kGrpStages;
+  void (*fn)(GemmArgs);
+  if constexpr (BIG) fn = gemm_grp_kernel<BM, kGrpBN, WM, kGrpWN, S, EPI, kGrpBK>;
+  else fn = gemm_kernel<BM, kGrpBN, WM, kGrpWN, S, EPI, false, true, kGrpBK>;
+  const size_t lds = std::max({(size_t)S * (BM + kGrpBN) * kGrpBK * 2, gemm_stage_bytes(BM, kGrpBN),
+                               gemm_stage_bytes(kGrpBN, BM)});
   constexpr int threads = 64 * WM * kGrpWN;
   if (hi_blocks_per_cu(reinterpret_cast<const void*>(fn), threads, lds) <= 0) HI_FAIL("moe: grouped GEMM does not fit");
-  const int tiles_n = (N + kGrpBN - 1) / kGrpBN;
-  hipLaunchKernelGGL(fn, dim3(max_row_tiles * tiles_n), dim3(threads), lds, s, g);
+  // the worst case of either shape: each expert adds at most one partial row tile
+  auto blocks = [&](int bm, int bn) { return ((n + bm - 1) / bm + E) * ((N + bn - 1) / bn); };
+  const int grid = BIG ? std::max(blocks(BM, kGrpBN), blocks(kGrpBN, BM)) : blocks(BM, kGrpBN);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(threads), lds, s, g);
   HI_TRY(hipGetLastError());
   return 0;
 }
@@ -528,7 +563,7 @@ int gemv_max() { return hi_gemv_max_rows(); }
 
 // The expert workspace (hi_moe_work_bytes), each piece on a 256-byte boundary. The first
 // kMoeBarBytes (at a fixed offset, whatever M) hold the one-token launch's arrival counters, which no
-// other launch uses; then perm [n], off and tiles [E+1] int, y [n, H] (pair order)
+// other launch uses; then perm [n], off [E+1] and tiles [E+2] int, y [n, H] (pair order)
 // and act [n, I] fp16 (sorted order on the grouped path, pair order on the GEMV path).
 constexpr int kMoeBarStride = 64;                 // words between two arrival counters (256 bytes)
 constexpr size_t kMoeBarBytes = 9 * 256;          // 8 counters, then the 8 expected totals
@@ -543,23 +578,25 @@ MoeWork moe_work(void* work, int n, int E, int H) {
   m.bar = (unsigned*)p; p += kMoeBarBytes;
   m.perm = (int*)p;   p += al256((size_t)n * 4);
   m.off = (int*)p;    p += al256((size_t)(E + 1) * 4);
-  m.tiles = (int*)p;  p += al256((size_t)(E + 1) * 4);
+  m.tiles = (int*)p;  p += al256((size_t)(E + 2) * 4);
   m.y = (f16*)p;      p += al256((size_t)n * H * 2);
   m.act = (f16*)p;
   return m;
 }
 
-// Row tile of the grouped GEMMs: 256 rows where the experts average 112 rows or more and 256-row tiles
-// still give every CU a block in both GEMMs. An expert of 129-256 rows is then one tile, its weights
-// streamed once, instead of two that are 30 % padding; a smaller grid would leave CUs idle. Measured,
-// whole layer, 128-row tiles -> 256: 32 experts, top 8, H 1024, I 512: 512 tokens 68.2 -> 62.9 us, 700
-// 75.7 -> 71.3, 2048 157.8 -> 148.0; 64 experts, top 6, H 2048, I 768: 1400 tokens 268.7 -> 249.8, 2048
-// 344.6 -> 287.3. The line: evenly routed experts of 100 rows on average all fit 128 rows and
-// are slower in 256 (400 tokens 48.8 -> 54.4); of 120 some do not, and their second tiles start another
-// round (448 tokens 68.1 -> 58.3, 480 66.9 -> 56.4). What bounds the GEMMs is their ring's start and end (16 and 8 K tiles) per round.
-bool moe_tall(int n, int E, int H, int I, int cus) {
+// Whether the grouped GEMMs take the big tiles: where the experts average more than 128 rows, so that some
+// expert needs a second row tile of 128 whatever the routing, and 256-row tiles still give every CU a block
+// in both GEMMs (a smaller grid would leave CUs idle). An expert of 129-256 rows is then one tile of 256, its
+// weights streamed once, or the columns are twice as wide (big_tiles_turned); what bounds the GEMMs is their
+// ring's start and end (16 and 8 K tiles) per round of blocks. Measured, whole layer, 128 x 128 tiles -> big,
+// evenly routed and in proportion to 1 / sqrt(rank), us: 32 experts, top 8, H 1024, I 512: 600 tokens 63.6 ->
+// 52.6 and 62.1 -> 53.6, 2048 140 -> 122 and 142 -> 124; 64 experts, top 6, H 2048, I 768: 1400 tokens 233 ->
+// 207 and 231 -> 221, 2048 297 -> 229 and 293 -> 255; 8, top 2, H 4096, I 14336: 520 tokens 862 -> 738 and 787 ->
+// 699. Below the line the routing decides: 448 tokens of the 32 experts take 50 to 56 us with the big tiles, and
+// with 128 x 128 47 where every expert fits 128 rows (one round of blocks), 58 to 61 where some do not.
+bool moe_big_tiles(int n, int E, int H, int I, int cus) {
   const int row_tiles = std::max(E, n / kGrpTallBM), tiles_n = (std::min(2 * I, H) + kGrpBN - 1) / kGrpBN;
-  return n / 112 >= E && (int64_t)row_tiles * tiles_n >= cus;
+  return n > kGrpBM * E && (int64_t)row_tiles * tiles_n >= cus;
 }
 
 // The grouped path: the sort (perm / off / tiles in wk), gate/up + SwiGLU on the rows of xn gathered by
@@ -572,18 +609,17 @@ int moe_grouped(const f16* xn, int ldxn, const f16* Wgu, const f16* Wd, const in
   // the tile DMA addresses xn's gathered rows, and act's and y's rows, at 32-bit byte offsets
   if ((int64_t)M * ldxn * 2 >= INT32_MAX || (int64_t)n * (H > I ? H : I) * 2 >= INT32_MAX)
     HI_FAIL("moe: %d rows too many for the grouped path's 32-bit offsets", M);
-  const bool tall = moe_tall(n, E, H, I, d->cus);
-  const int bm = tall ? kGrpTallBM : kGrpBM;
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kSortThreads), 0, st, idx, n, E, bm, wk.off, wk.tiles, wk.perm);
+  const bool big = moe_big_tiles(n, E, H, I, d->cus);
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kSortThreads), 0, st, idx, n, E, big ? kGrpTallBM : kGrpBM, H, I,
+                     d->cus, wk.off, wk.tiles, wk.perm);
   HI_TRY(hipGetLastError());
-  const int max_row_tiles = (n + bm - 1) / bm + E;  // each expert adds at most one partial tile
-  const auto gu = tall ? grouped_gemm<2, kGrpTallBM, kGrpTallWM, kGrpTallStages> : grouped_gemm<2, kGrpBM, kGrpWM, kGrpStages>;
-  const auto down = tall ? grouped_gemm<0, kGrpTallBM, kGrpTallWM, kGrpTallStages> : grouped_gemm<0, kGrpBM, kGrpWM, kGrpStages>;
+  const auto gu = big ? grouped_gemm<2, true> : grouped_gemm<2, false>;
+  const auto down = big ? grouped_gemm<0, true> : grouped_gemm<0, false>;
   if (int r = gu(xn, ldxn, M, Wgu, (int64_t)2 * I * H * 2, wk.act, I, 2 * I, H, wk.off, wk.tiles, wk.perm, k, true, false,
-                 E, max_row_tiles, st))
+                 E, n, st))
     return r;
-  if (int r = down(wk.act, I, n, Wd, (int64_t)H * I * 2, wk.y, H, H, I, wk.off, wk.tiles, wk.perm, 1, false, true, E,
-                   max_row_tiles, st))
+  if (int r = down(wk.act, I, n, Wd, (int64_t)H * I * 2, wk.y, H, H, I, wk.off, wk.tiles, wk.perm, 1, false, true, E, n,
+                   st))
     return r;
   const auto comb = k <= 4 ? moe_combine_kernel<4> : k <= 8 ? moe_combine_kernel<8> : moe_combine_kernel<16>;
   hipLaunchKernelGGL(comb, dim3(M), dim3(128), 0, st, wk.y, idx, w, k, E, H, flags, scale, x, (int64_t)ldx);
@@ -927,7 +963,8 @@ HI_EXPORT int hi_moe_router(const void* xn, int ldx, const void* Wr, int M, int 
 // path uses only act.
 HI_EXPORT size_t hi_moe_work_bytes(int M, int k, int E, int H, int I) {
   const size_t n = (size_t)(M > 0 ? M : 0) * (k > 0 ? k : 0);
-  return kMoeBarBytes + al256(n * 4) + 2 * al256((size_t)(E + 1) * 4) + al256(n * H * 2) + al256(n * I * 2);
+  return kMoeBarBytes + al256(n * 4) + al256((size_t)(E + 1) * 4) + al256((size_t)(E + 2) * 4) + al256(n * H * 2) +
+         al256(n * I * 2);
 }
 
 // x[m] += MoE(xn[m]) for M rows given the routing (idx, w from hi_moe_router): wgu [E][2I, H]

@@ -108,26 +108,55 @@ def test_moe_grouped_path_graph_replay(hi, O):
         hi.moe_experts(xn_d, wgu_d, wdn_d, idx_d, w_d, cuda(x0), flags, 0.22, 2)  # eager work between replays
 
 
+UNEVEN = [0, 1, 127, 128, 129, 255, 256, 257, 511, 512, 513] + [90] * 21   # rows per expert
+WITHIN_256 = [0, 1, 127, 128, 129, 255, 256] + [150] * 25
+
+
+@pytest.mark.parametrize("counts,turned", [(UNEVEN, 1), (WITHIN_256, 0)], ids=["uneven", "within_256"])
 @pytest.mark.parametrize("H,I", [(1024, 512), (1056, 544)])
-def test_moe_grouped_tall_tiles_bit_identical(hi, H, I):
-    """112 rows per expert on average and more take the 256-row tiles, whose sums run in the 128-row tiles'
-    order: experts of no row, of one, and of either tile's edges, against calls of 400 tokens (the
-    128-row tiles, checked against the oracle above), bit for bit."""
+def test_moe_grouped_tall_tiles_bit_identical(hi, H, I, counts, turned):
+    """More than 128 rows per expert on average take the big tiles: 256 x 128, or 128 x 256 where those make
+    fewer rounds of blocks (here where a few experts are over 256 rows). Their sums run in the 128 x 128
+    tiles' order: experts of no row, of one, and of every tile's edges, against calls of 400 tokens (the
+    128 x 128 tiles, checked against the oracle above), bit for bit. The sort leaves the shape behind the
+    row-tile prefix in the work buffer."""
+    import torch
     r = rng(440 + H)
-    E, flags = 32, 1
-    counts = [0, 1, 127, 128, 129, 255, 256, 257, 511, 512, 513] + [90] * 21
+    E, flags, cus = 32, 1, hi.lib.hi_device_cus()
     ids = np.concatenate([np.full(c, e) for e, c in enumerate(counts)] + [[-1, E]]).astype(np.int32)
     r.shuffle(ids)
     M = len(ids)
-    assert (M - 2) // 112 >= E
+    assert M > 128 * E and E * -(-min(2 * I, H) // 128) >= cus, "the big tiles' rule"
     wgu, wdn = cuda(rn(r, E, 2 * I, H, s=0.02)), cuda(rn(r, E, H, I, s=0.02))
     xn, x0, idx = cuda(rn(r, M, H)), cuda(rn(r, M, H)), cuda(ids[:, None])
     w = cuda(r.random((M, 1)).astype(np.float32))
-    got = host(hi.moe_experts(xn, wgu, wdn, idx, w, x0.clone(), flags, 0.22, 2))
+    x = x0.clone()
+    work = torch.empty(hi.lib.hi_moe_work_bytes(M, 1, E, H, I), dtype=torch.uint8, device="cuda")
+    hi.check_rc(hi.lib.hi_moe_experts(hi.ptr(xn), H, hi.ptr(wgu), hi.ptr(wdn), hi.ptr(idx), hi.ptr(w), M, E, 1, H, I,
+                                      flags, 0.22, hi.ptr(x), H, 2, hi.ptr(work), hi.cur_stream()), "moe_experts")
+    if cus == 256:  # the shape's rounds are those of 256 CUs
+        al = lambda n: -(-n // 256) * 256
+        at = 9 * 256 + al(4 * M) + al(4 * (E + 1)) + 4 * (E + 1)
+        assert int(work[at:at + 4].view(torch.int32)) == turned
+    got = host(x)
     for a in range(0, M, 400):
         b = slice(a, min(a + 400, M))
         ref = host(hi.moe_experts(xn[b], wgu, wdn, idx[b], w[b], x0[b].clone(), flags, 0.22, 2))
         assert np.array_equal(got[b].view(np.uint16), ref.view(np.uint16)), f"rows {a}.."
+
+
+def test_moe_grouped_tall_tiles_top8_prompt(hi, O):
+    """The router, the gather by token and the combine of eight slots around the big tiles: a 520-token prompt of
+    a 32-expert layer (130 rows per expert) against the oracle."""
+    r = rng(450)
+    E, k, H, I, flags, M = 32, 8, 1024, 512, 3, 520
+    assert M * k > 128 * E and E * (H // 128) >= hi.lib.hi_device_cus(), "the big tiles' rule"
+    Wr, wgu, wdn = rn(r, E, H, s=0.05), rn(r, E, 2 * I, H, s=0.02), rn(r, E, H, I, s=0.02)
+    xn, x0 = rn(r, M, H), rn(r, M, H)
+    x = cuda(x0)
+    idx, w = hi.moe_route_experts(cuda(xn), cuda(Wr), cuda(wgu), cuda(wdn), k, x, flags, 0.22)
+    check("moe 520 tokens top 8", host(x), O.moe_experts(xn, wgu, wdn, host(idx), host(w), x0.copy(), flags, 0.22),
+          4e-3, 4e-3)
 
 
 def test_moe_out_of_range_expert_ids_contribute_nothing(hi, O):
