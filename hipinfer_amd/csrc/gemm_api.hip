@@ -486,7 +486,13 @@ HI_EXPORT int hi_gemm_last_choice(int* cfg, int* splits) {
 }
 HI_EXPORT int hi_gemm_config_desc(int c, char* out, int n) {
   if (c < 0 || c >= kGemmNumCfgs || !out || n < 1) return -1;
-  snprintf(out, n, "mfma 32x32x16 %dx%dx%d waves %dx%dx%d stages %d", kGemmCfgs[c].bm, kGemmCfgs[c].bn, kGemmCfgs[c].bk,
-           kGemmCfgs[c].wm, kGemmCfgs[c].wn, kGemmCfgs[c].kg, kGemmCfgs[c].st);
+  const GemmCfg& k = kGemmCfgs[c];
+  char st[48];  // ring stages, A's and W's apart where they differ
+  if (gemm_sa(c, false) == gemm_sb(c, false))
+    snprintf(st, sizeof st, "%d", k.st);
+  else
+    snprintf(st, sizeof st, "%d A, %d W (int8: %d A, %d W)", gemm_sa(c, false), gemm_sb(c, false), gemm_sa(c, true),
+             gemm_sb(c, true));
+  snprintf(out, n, "mfma 32x32x16 %dx%dx%d waves %dx%dx%d stages %s", k.bm, k.bn, k.bk, k.wm, k.wn, k.kg, st);
   return 0;
 }

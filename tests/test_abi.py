@@ -33,6 +33,26 @@ def test_library_loads_and_resolves_every_symbol():
         assert getattr(lib, name) is not None
 
 
+def test_gemm_config_desc_states_the_ring():
+    """The 64-deep tiles of 256 rows by 192 or 256 columns hold one W stage more than A stages, and with int8
+    weights one of each more still; the others as many of both."""
+    lib = ctypes.CDLL(LIB)
+    buf = ctypes.create_string_buffer(128)
+    uneven = 0
+    for cfg in range(lib.hi_gemm_num_configs()):
+        assert lib.hi_gemm_config_desc(cfg, buf, 128) == 0
+        m = re.fullmatch(r"mfma 32x32x16 (\d+)x(\d+)x(\d+) waves \d+x\d+x\d+ stages (.+)", buf.value.decode())
+        bm, bn, bk = int(m[1]), int(m[2]), int(m[3])
+        if bm == 256 and bn >= 192 and bk == 64:
+            uneven += 1
+            assert m[4] == "2 A, 3 W (int8: 3 A, 4 W)"
+            for a, w, row in ((2, 3, 2), (3, 4, 1)):  # both rings fit a CU's 160 KB
+                assert bk * (a * bm * 2 + w * bn * row) <= 160 * 1024
+        else:
+            assert re.fullmatch(r"[2-8]", m[4])
+    assert uneven == 3
+
+
 def test_library_holds_gfx950_code_objects():
     blob = open(LIB, "rb").read()
     assert b"gfx950" in blob
