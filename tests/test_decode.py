@@ -68,9 +68,10 @@ def test_decode_attn_batch64(hi, O):
 @pytest.mark.parametrize("D,Hkv,G", [(64, 8, 8), (128, 8, 4), (128, 2, 5)], ids=["D64-G8", "D128-G4", "D128-G5"])
 @pytest.mark.parametrize("B", [1, 3, 24, 70], ids=lambda b: f"B{b}")
 def test_decode_attn_tile_and_split_edges(hi, O, D, Hkv, G, B):
-    """Lengths at the edges of a wave's 32 keys, a block pass of 4 or 8 waves (128 and 256 keys) and
-    the split rule's steps (128, 256 and 1024 keys, 16 splits), at batches of both block widths, with
-    infinities and NaN in the cache behind every length: keys past it must not take part."""
+    """Lengths at the edges of a wave's 32 keys, of 128 and 256 keys (a pass of a block of 4 and of 8 waves where one
+    split runs) and of the split rule's steps up to 16 splits, at batches of both block widths, with
+    infinities and NaN in the cache behind every length: keys past it must not take part. Runs of several
+    tiles a wave and more than 16 splits: test_decode_attn_long_contexts."""
     edges = [1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 1023, 1024, 1025, 2047, 2048, 2049, 2079, 2080]
     S, Hq = 2080, Hkv * G
     for first in range(len(edges) if B == 1 else 1):
@@ -87,6 +88,26 @@ def test_decode_attn_tile_and_split_edges(hi, O, D, Hkv, G, B):
         pos = np.array(lens, np.int32) - 1
         got = host(hi.decode_attn(cuda(q), cuda(kc), cuda(vc), cuda(pos), Hq, Hkv))
         check(f"decode attn D={D} G={G} B={B} lens={lens[:4]}", got, O.decode_attn(q, kc, vc, pos, Hq, Hkv), 2e-3, 1e-2)
+
+
+@pytest.mark.parametrize("D,Hkv,G", [(64, 8, 4), (128, 8, 4), (128, 2, 6)], ids=["D64-G4", "D128-G4", "D128-Hkv2"])
+@pytest.mark.parametrize("lens", [[4097], [6000], [8500], [4096, 4097, 4352, 6000], [6100, 33, 2500]],
+                         ids=lambda l: "-".join(map(str, l)))
+def test_decode_attn_long_contexts(hi, O, D, Hkv, G, lens):
+    """Blocks of 8 waves whose waves run several tiles (splits of over 256 keys), and merges of more than the 16
+    splits that one round requests (17 to 34 at batch 1), with infinities and NaN in the cache behind every
+    length."""
+    r = rng(670 + len(lens) + lens[0] + D)
+    B, S, Hq = len(lens), max(lens) + 32, Hkv * G
+    q = r.standard_normal((B, Hq * D)).astype(np.float16)
+    kc = r.standard_normal((B, Hkv, S, D)).astype(np.float16)
+    vc = r.standard_normal((B, Hkv, S, D)).astype(np.float16)
+    for b, n in enumerate(lens):
+        kc[b, :, n:] = np.inf
+        vc[b, :, n:] = np.nan
+    pos = np.array(lens, np.int32) - 1
+    got = host(hi.decode_attn(cuda(q), cuda(kc), cuda(vc), cuda(pos), Hq, Hkv))
+    check(f"decode attn D={D} G={G} lens={lens}", got, O.decode_attn(q, kc, vc, pos, Hq, Hkv), 2e-3, 1e-2)
 
 
 @pytest.mark.parametrize("D,Hkv,G", [(64, 4, 8), (128, 8, 4)], ids=["D64-G8", "D128-G4"])

@@ -291,6 +291,24 @@ def test_gemm_short_k(hi, O):
         hi.lib.hi_gemm_force_splits(-1)
 
 
+def test_gemm_int8_short_k(hi, O):
+    """int8 weights with fewer K tiles than any ring has stages and up to one more than the deepest 64-deep one
+    (3 A and 4 W stages on the 256-row tiles by 192 and 256 columns), with and without a K tail of 32."""
+    r = rng(335)
+    try:
+        for cfg in CFGS:
+            hi.lib.hi_gemm_force_config(cfg)
+            hi.lib.hi_gemm_force_splits(1)
+            for K in [32, 64, 96, 128, 160, 192, 224, 256, 288, 320]:
+                M = 300 if K % 64 else 70
+                q, s = O.quantize_rows(h16(r, 1024, K, sd=0.02))
+                gemm_check(hi, O, f"int8 short-K cfg={cfg} K={K}", h16(r, M, K), q, r, scales=s)
+                assert_ran(hi, cfg, True, K, f"int8 short-K K={K}")
+    finally:
+        hi.lib.hi_gemm_force_config(-1)
+        hi.lib.hi_gemm_force_splits(-1)
+
+
 @pytest.mark.parametrize("cfg", CFGS)
 def test_gemm_int8(hi, O, cfg):
     need_cfg(hi, cfg)
