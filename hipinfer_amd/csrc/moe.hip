@@ -959,7 +959,7 @@ HI_EXPORT int hi_moe_router(const void* xn, int ldx, const void* Wr, int M, int 
 }
 
 // Expert workspace, each piece on a 256-byte boundary: arrival counters (2304 bytes, first,
-// whatever M), perm [M*k] int, off, tiles [E+1] int, y [M*k, H] and act [M*k, I] fp16. The GEMV
+// whatever M), perm [M*k] int, off [E+1], tiles [E+2] int, y [M*k, H] and act [M*k, I] fp16. The GEMV
 // path uses only act.
 HI_EXPORT size_t hi_moe_work_bytes(int M, int k, int E, int H, int I) {
   const size_t n = (size_t)(M > 0 ? M : 0) * (k > 0 ? k : 0);
@@ -1006,8 +1006,9 @@ HI_EXPORT int hi_moe_experts(const void* xn, int ldxn, const void* wgu, const vo
 // hi_moe_experts with path 0. One row runs as one launch (moe_decode_one_kernel) when its grid fits
 // on the GPU at once; otherwise, on the GEMV path (M <= HIPINFER_GEMV_MAX), the router runs inside
 // the gate/up launch (moe_route_gu_kernel), which saves a launch and a dependent memory round trip
-// per layer; larger M run the router and the grouped experts as two calls. The work buffer must be
-// zeroed once before its first use here (its arrival counters; every call leaves them consistent).
+// per layer; larger M run the router and the grouped experts as two calls. The first kMoeBarBytes of
+// the work buffer must be zeroed once before the first one-row call (its arrival counters; every call
+// leaves them consistent); more rows use no counters and take any buffer.
 // No counterpart in the reference, whose engine makes the two calls (api.cu:1701-1703); this
 // build's engine uses this.
 HI_EXPORT int hi_moe_route_experts(const void* xn, int ldxn, const void* Wr, const void* wgu, const void* wdown, int M,

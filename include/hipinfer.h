@@ -96,8 +96,8 @@ int hi_gemm_residual_rmsnorm(const void* A, int lda, const void* W, const void* 
  * Replaces api.cu:849-857 (hi_moe_router); hipinfer.py:68. */
 int hi_moe_router(const void* xn, int ldx, const void* Wr, int M, int E, int H, int k, int flags, int* idx, float* w,
                   void* stream);
-/* Bytes of the workspace hi_moe_experts and hi_moe_route_experts need (the first 2304 bytes hold
- * hi_moe_route_experts' arrival counters). Replaces api.cu:862-865 (hi_moe_work_bytes); hipinfer.py:69. */
+/* Bytes of the workspace hi_moe_experts and hi_moe_route_experts need (the first 2304 bytes hold the
+ * arrival counters of hi_moe_route_experts with M = 1). Replaces api.cu:862-865 (hi_moe_work_bytes); hipinfer.py:69. */
 size_t hi_moe_work_bytes(int M, int k, int E, int H, int I);
 /* x[m] += MoE(xn[m]) given the routing: wgu [E][2I, H] (gate/up interleaved per expert), wdown [E][H, I];
  * scale multiplies the combined output (rounded); path 0 auto (GEMV for M <= HIPINFER_GEMV_MAX, default 8),
@@ -110,9 +110,10 @@ int hi_moe_experts(const void* xn, int ldxn, const void* wgu, const void* wdown,
  * idx[M, k] / w[M, k] as hi_moe_router writes it; the same bits as hi_moe_router followed by
  * hi_moe_experts(path 0). M = 1 runs as one launch (router, gate/up, a grid-wide handoff, down and
  * combine) when that grid fits on the GPU at once; otherwise, for M <= HIPINFER_GEMV_MAX, the router
- * runs inside the gate/up launch. work: hi_moe_work_bytes(M, k, E, H, I), zeroed once before its
- * first use with this function (the one-launch path keeps arrival counters in it and leaves them
- * consistent); calls that share a work buffer must not overlap in time. Returns -2, launching
+ * runs inside the gate/up launch. work: hi_moe_work_bytes(M, k, E, H, I); its first 2304 bytes zeroed
+ * once before the first call with M = 1 (the one-launch path keeps arrival counters there and leaves
+ * them consistent; larger M neither reads nor writes them, so its buffer may hold anything); calls
+ * that share a work buffer must not overlap in time. Returns -2, launching
  * nothing, when an earlier one-launch call gave up waiting for its grid (its output was wrong; the
  * one-launch path is then off for the rest of the process).
  * No counterpart in the reference (its engine makes the two calls, api.cu:1701-1703); for callers

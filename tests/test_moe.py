@@ -283,6 +283,29 @@ def test_moe_route_experts_grouped_graph_replay(hi):
         assert np.array_equal(host(xe).view(np.uint16), ref.view(np.uint16))
 
 
+@pytest.mark.parametrize("M", [2, 8, 9, 200])
+def test_moe_route_experts_needs_no_zeroed_work_past_one_row(hi, M):
+    """Only the one-row launch uses arrival counters: with more rows a work buffer of any content gives the same
+    bits, and the counters' 2304 bytes stay as they were."""
+    import torch
+    r = rng(470 + M)
+    E, k, H, I, flags = 32, 8, 512, 256, 3
+    Wr, wgu, wdn = cuda(rn(r, E, H, s=0.05)), cuda(rn(r, E, 2 * I, H, s=0.02)), cuda(rn(r, E, H, I, s=0.02))
+    xn, x0 = cuda(rn(r, M, H)), cuda(rn(r, M, H))
+    idx = torch.empty(M, k, dtype=torch.int32, device="cuda")
+    w = torch.empty(M, k, dtype=torch.float32, device="cuda")
+    out = []
+    for fill in (0, 0x5A, 0xFF):
+        x = x0.clone()
+        work = torch.full((hi.lib.hi_moe_work_bytes(M, k, E, H, I),), fill, dtype=torch.uint8, device="cuda")
+        hi.check_rc(hi.lib.hi_moe_route_experts(hi.ptr(xn), H, hi.ptr(Wr), hi.ptr(wgu), hi.ptr(wdn), M, E, k, H, I, flags,
+                                                0.22, hi.ptr(x), H, hi.ptr(idx), hi.ptr(w), hi.ptr(work), hi.cur_stream()),
+                    "moe_route_experts")
+        assert (work[:2304] == fill).all()
+        out.append(host(x).view(np.uint16))
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+
+
 def test_moe_route_experts_shared_work_across_shapes(hi):
     """One zeroed work buffer serves single-row calls of every layer shape in turn, twice round:
     the one-launch path's arrival counters live in it and carry each launch's totals to the next
