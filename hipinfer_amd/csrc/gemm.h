@@ -143,30 +143,49 @@ __device__ __forceinline__ void sched_step() {
   for (; v < NV; v++) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
 }
 
+// Grouped mode: what a thread loads of the groups before anything else (thread e < grp_n its group's tile
+// start and first row, thread 0 also the totals).
+struct GrpLoad {
+  int tile, off, tiles_all, off_all;
+};
+__device__ __forceinline__ GrpLoad grp_load(const GemmArgs& g) {
+  GrpLoad l{};
+  const int tid = threadIdx.x;
+  if (tid < g.grp_n) {
+    l.tile = g.grp_tiles[tid];
+    l.off = g.grp_off[tid];
+  }
+  if (tid == 0) {
+    l.tiles_all = g.grp_tiles[g.grp_n];
+    l.off_all = g.grp_off[g.grp_n];
+  }
+  return l;
+}
+
 template <int BM, int BN, int WM, int WN, int S, int EPI, bool Q8, bool GRP = false, int BK = 64, int KG = 1, int SB = S>
 __global__ void __launch_bounds__(64 * WM * WN * KG) gemm_kernel(GemmArgs g) {
+  constexpr bool PRELOADED = false;
+  constexpr GrpLoad loaded{};
 #include "gemm_body.h"
 }
 
 // Grouped mode with the tile's shape chosen on the device, which knows the groups' sizes: BM x BN or, where
-// grp_tiles[grp_n + 1] is not 0, BN x BM (and WN x WM waves: the wave tile, the ring and the order of the sums
-// are the same). The groups' tables are requested together with that word, so that the body finds them in
-// the cache and the choice costs no second round trip to memory.
+// grp_tiles[grp_n + 1] is not 0, BN x BM (and WN x WM waves; the wave tile, the ring and the order of the sums
+// are the same). That word is loaded with the groups, so the choice costs no round trip of its own.
 template <int BM, int BN, int WM, int WN, int S, int EPI, int BK>
-__device__ __forceinline__ void gemm_grp_shape(GemmArgs g) {
-  constexpr bool Q8 = false, GRP = true;
+__device__ __forceinline__ void gemm_grp_shape(GemmArgs g, GrpLoad loaded) {
+  constexpr bool Q8 = false, GRP = true, PRELOADED = true;
   constexpr int KG = 1, SB = S;
 #include "gemm_body.h"
 }
 template <int BM, int BN, int WM, int WN, int S, int EPI, int BK>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_grp_kernel(GemmArgs g) {
-  const int tid = threadIdx.x, tables = tid <= g.grp_n ? g.grp_tiles[tid] ^ g.grp_off[tid] : 0;
   const int turned = g.grp_tiles[g.grp_n + 1];
-  asm volatile("" ::"v"(tables));
+  const GrpLoad loaded = grp_load(g);
   if (turned == 0)
-    gemm_grp_shape<BM, BN, WM, WN, S, EPI, BK>(g);
+    gemm_grp_shape<BM, BN, WM, WN, S, EPI, BK>(g, loaded);
   else
-    gemm_grp_shape<BN, BM, WN, WM, S, EPI, BK>(g);
+    gemm_grp_shape<BN, BM, WN, WM, S, EPI, BK>(g, loaded);
 }
 
 // Split-K second pass: sum the fp32 partials [splits][M][N] in split order (deterministic) and run

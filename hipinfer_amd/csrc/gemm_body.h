@@ -1,7 +1,8 @@
-// The body of the GEMM kernels (gemm.h includes it inside each of their functions): template parameters
-// BM, BN, WM, WN, S, EPI, Q8, GRP, BK, KG, SB, argument g. One text and not one inlined function: as a
-// function, the compiler ordered the same code differently in every instance, up to 10 % slower (256 x 192,
-// M = 2048, N = 4096, K = 14336: 239 -> 264 us; 128 x 96, M = 777, N = 2560, K = 2048: 15.9 -> 17.2).
+// The body of the GEMM kernels; gemm.h includes it in each of their functions. It uses their template parameters
+// BM, BN, WM, WN, S, EPI, Q8, GRP, BK, KG, SB, the argument g and, where PRELOADED, the thread's GrpLoad `loaded`.
+// One text and not one inlined function: as a function, the compiler ordered the same code differently in every
+// instance, up to 10 % slower (256 x 192, M = 2048, N = 4096, K = 14336: 239 -> 264 us; 128 x 96, M = 777, N =
+// 2560, K = 2048: 15.9 -> 17.2).
   constexpr int TM = BM / WM, TN = BN / WN;          // wave tile
   constexpr int FM = TM / 32, FN = TN / 32;          // MFMA tiles per wave
   constexpr int A_ST = BM * BK;                      // halves per stage
@@ -63,24 +64,22 @@
   if constexpr (GRP) {
     // find this block's group: grp_tiles[e] <= row tile < grp_tiles[e + 1] (the prefix is
     // non-decreasing, so e is the number of groups whose tiles start at or before the row tile,
-    // minus one); blocks past the last row tile (the grid is sized for the worst case) exit. Every
-    // thread loads one group's tile start and first row at once (thread 0 also the totals): one
-    // memory round trip, then one counting barrier.
+    // minus one); blocks past the last row tile (the grid is sized for the worst case) exit. The threads
+    // load the groups at once (grp_load): one memory round trip, then one counting barrier.
     static_assert(64 * NW * KG >= kGemmMaxGroups, "one thread per group");
     __shared__ int s_tiles[kGemmMaxGroups + 1], s_off[kGemmMaxGroups + 1];
     const int E = g.grp_n, mt = blockIdx.x / tiles_n;
     tn = blockIdx.x - mt * tiles_n;
-    int te = 0;
+    const GrpLoad gl = PRELOADED ? loaded : grp_load(g);
     if (tid < E) {
-      te = g.grp_tiles[tid];
-      s_tiles[tid] = te;
-      s_off[tid] = g.grp_off[tid];
+      s_tiles[tid] = gl.tile;
+      s_off[tid] = gl.off;
     }
     if (tid == 0) {
-      s_tiles[E] = g.grp_tiles[E];
-      s_off[E] = g.grp_off[E];
+      s_tiles[E] = gl.tiles_all;
+      s_off[E] = gl.off_all;
     }
-    const int lo = __syncthreads_count(tid < E && te <= mt) - 1;
+    const int lo = __syncthreads_count(tid < E && gl.tile <= mt) - 1;
     if (mt >= s_tiles[E]) return;
     grp_r0 = s_off[lo];
     M = s_off[lo + 1] - grp_r0;
