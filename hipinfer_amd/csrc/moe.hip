@@ -359,18 +359,20 @@ __global__ void __launch_bounds__(kMoeWaves * 64) moe_gemv_down_kernel(const f16
 constexpr int kSortThreads = 1024;
 
 // Whether the big tiles should be 128 rows x 256 columns rather than 256 x 128, for experts that come to t256
-// and t128 row tiles: where the GEMMs' blocks (gate/up [2I, H], down [H, I]; one per CU) make less rounds of
-// them, a round taking its K tiles and about 8 for the ring's start and end. 256 rows stream an expert of
-// up to 256 once, but experts over 256 rows, as uneven routing makes them, bring a few row tiles of 256 and
-// with them a part-filled second round; 128 rows also waste less on them. 32 experts, top 8, H 1024, I 512,
-// experts chosen in proportion to 1 / sqrt(rank), 256 x 128 / 128 x 256 / 128 x 128 with 4 waves, us: 600 tokens
-// 71.5 / 53.6 / 62.1, 700 73.8 / 57.6 / 64.8, 64 experts, top 6, H 2048, I 768: 1400 tokens 228.9 / 221.0 / 231.1.
+// and t128 row tiles: where the GEMMs' blocks (gate/up [2I, H], down [H, I]; one per CU) make an eighth less
+// rounds of them, a round taking its K tiles and about 8 for the ring's start and end. 256 rows stream an
+// expert of up to 256 once, but experts over 256 rows, as uneven routing makes them, bring a few row tiles of
+// 256 and with them a part-filled second round; 128 rows also waste less on them. Within an eighth the weights,
+// streamed once more per extra row tile, count for more. 32 experts, top 8, H 1024, I 512, experts chosen in
+// proportion to 1 / sqrt(rank), 256 x 128 / 128 x 256 / 128 x 128 with 4 waves, us: 600 tokens 71.5 / 53.6 / 62.1,
+// 700 73.8 / 57.6 / 64.8; 64, top 6, H 2048, I 768: 1400 tokens 228.9 / 221.0 / 231.1; 8, top 2, H 4096, I 14336,
+// 520 tokens in proportion to 1 / rank (36 % less rounds) 819 / 740 / 815, evenly (10 % less) 693 / 767 / 868.
 __device__ bool big_tiles_turned(int t256, int t128, int H, int I, int cus) {
   auto rounds = [&](int row_tiles, int bn, int N) { return (row_tiles * ((N + bn - 1) / bn) + cus - 1) / cus; };
   auto cost = [&](int row_tiles, int bn) {
     return rounds(row_tiles, bn, 2 * I) * (H / kGrpBK + 8) + rounds(row_tiles, bn, H) * (I / kGrpBK + 8);
   };
-  return cost(t128, kGrpTallBM) < cost(t256, kGrpBN);
+  return 8 * cost(t128, kGrpTallBM) < 7 * cost(t256, kGrpBN);
 }
 
 __global__ void __launch_bounds__(kSortThreads) moe_sort_kernel(const int* __restrict__ idx, int n, int E,
@@ -591,8 +593,8 @@ MoeWork moe_work(void* work, int n, int E, int H) {
 // ring's start and end (16 and 8 K tiles) per round of blocks. Measured, whole layer, 128 x 128 tiles -> big,
 // evenly routed and in proportion to 1 / sqrt(rank), us: 32 experts, top 8, H 1024, I 512: 600 tokens 63.6 ->
 // 52.6 and 62.1 -> 53.6, 2048 140 -> 122 and 142 -> 124; 64 experts, top 6, H 2048, I 768: 1400 tokens 233 ->
-// 207 and 231 -> 221, 2048 297 -> 229 and 293 -> 255; 8, top 2, H 4096, I 14336: 520 tokens 862 -> 738 and 787 ->
-// 699. Below the line the routing decides: 448 tokens of the 32 experts take 50 to 56 us with the big tiles, and
+// 207 and 231 -> 221, 2048 297 -> 229 and 293 -> 255; 8, top 2, H 4096, I 14336: 520 tokens 868 -> 693 and 805 ->
+// 715. Below the line the routing decides: 448 tokens of the 32 experts take 50 to 56 us with the big tiles, and
 // with 128 x 128 47 where every expert fits 128 rows (one round of blocks), 58 to 61 where some do not.
 bool moe_big_tiles(int n, int E, int H, int I, int cus) {
   const int row_tiles = std::max(E, n / kGrpTallBM), tiles_n = (std::min(2 * I, H) + kGrpBN - 1) / kGrpBN;
