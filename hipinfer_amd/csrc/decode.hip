@@ -24,7 +24,7 @@
 //  * online softmax per wave, the block's waves merged through LDS;
 //  * measured, cold caches, against one key per lane with v_dot2 and K through LDS (56-64 KB of it, so
 //    two blocks per CU and no overlap of loads with arithmetic inside a wave), us: 48 sequences of 100
-//    to 2000 keys, 32/8 heads of 128: 49.6 -> 43.5; 64 of 1000: 53 -> 49.8 (5.3 TB/s); 40 of 200 to
+//    to 2000 keys, 32/8 heads of 128: 49.6 -> 43.5; 64 of 1000: 51.4 -> 47.2 (5.6 TB/s); 40 of 200 to
 //    1600, 32/4 heads of 64: 24.6 -> 15.4; one of 4001, 32/8 of 128: 11.7 -> 10.5; four of 700 to 800,
 //    32/4 of 64: 11.1 -> 7.4;
 //  * splits hand their partials (o, m, l) to the last-arriving block of their (sequence, kv head)
